@@ -4,13 +4,18 @@ The library (`_lib/libgpa_mi355x.so`, built by `gpa-vggt_amd/build.py`)
 exports the plain C ABI declared in `include/gpa_mi355x.h`.  This module
 binds it with ctypes *after* importing torch, so the library resolves
 `libamdhip64.so.7` to the HIP runtime torch already loaded, and registers
-two custom ops:
+the custom ops:
 
     gpa::sim_argmax(Tensor a, Tensor b) -> (Tensor max_f32, Tensor idx_i64)
     gpa::attn_keybias(Tensor q, Tensor k, Tensor v, Tensor? bias,
                       float sm_scale, bool return_lse) -> (Tensor o, Tensor lse)
     gpa::merge_heads(Tensor t, Tensor offsets, Tensor tokens, int slots,
                      bool mean) -> (Tensor out, Tensor size, Tensor log_size)
+    gpa::merge_order(Tensor? cell, int frames, int w, int h, int sx, int sy,
+                     int num_special, Device device) -> (Tensor mask, Tensor order)
+    gpa::merge_plan(Tensor node_max, Tensor node_idx, Tensor order, int num_dst,
+                    int r) -> (Tensor edge, Tensor dst_slot, Tensor unm_abs,
+                    Tensor src_abs, Tensor size, Tensor offsets, Tensor tokens)
     gpa::lse_combine(Tensor out_a, Tensor lse_a, Tensor out_b, Tensor lse_b,
                      int frames) -> Tensor y              (bf16 or fp16)
     gpa::qk_norm_rope(Tensor qkv, Tensor ln_w, Tensor ln_b, float eps,
@@ -33,7 +38,7 @@ from typing import Optional, Tuple
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libgpa_mi355x.so"
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 GPA_OK = 0
 GPA_E_INVALID = -1
@@ -149,6 +154,18 @@ def _bind(lib: ctypes.CDLL) -> None:
     ]
     lib.gpa_residual_layernorm_f16.restype = ctypes.c_int
     lib.gpa_residual_layernorm_f16.argtypes = lib.gpa_residual_layernorm_bf16.argtypes
+    lib.gpa_merge_order.restype = ctypes.c_int
+    lib.gpa_merge_order.argtypes = [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp]
+    lib.gpa_merge_plan_workspace_bytes.restype = ctypes.c_size_t
+    lib.gpa_merge_plan_workspace_bytes.argtypes = [_i64, _i64]
+    lib.gpa_merge_plan.restype = ctypes.c_int
+    lib.gpa_merge_plan.argtypes = [
+        _vp, ctypes.c_int, _vp, _vp,   # node_max, max_dtype, node_idx, order
+        _i64, _i64, _i64, _i64,        # B, N, num_dst, r
+        _vp, _vp, _vp, _vp,            # edge, dst_slot, unm_abs, src_abs
+        _vp, _vp, _vp,                 # size, offsets, tokens
+        _vp, ctypes.c_size_t, _vp,     # workspace, workspace_bytes, stream
+    ]
     lib.gpa_merge_heads.restype = ctypes.c_int
     lib.gpa_merge_heads.argtypes = [
         _vp, ctypes.c_int, _vp,        # t, dtype, out
@@ -184,7 +201,8 @@ def lib() -> ctypes.CDLL:
 def exported_symbols() -> Tuple[str, ...]:
     return ("gpa_abi_version", "gpa_last_error", "gpa_sim_argmax_workspace_bytes",
             "gpa_sim_argmax_bf16", "gpa_attn_keybias_workspace_bytes", "gpa_attn_keybias_bf16",
-            "gpa_merge_heads", "gpa_lse_combine_bf16", "gpa_qk_norm_rope_bf16",
+            "gpa_merge_heads", "gpa_merge_order", "gpa_merge_plan_workspace_bytes",
+            "gpa_merge_plan", "gpa_lse_combine_bf16", "gpa_qk_norm_rope_bf16",
             "gpa_pool_shared_bf16", "gpa_merge_metric_bf16", "gpa_sim_argmax_f16",
             "gpa_attn_keybias_f16", "gpa_residual_layernorm_bf16",
             "gpa_attn_keybias_bf16_noalloc", "gpa_lse_combine_f16", "gpa_qk_norm_rope_f16",
@@ -458,6 +476,85 @@ def _merge_heads_fake(t, offsets, tokens, slots, mean):
     B, H, N, D = t.shape
     return (t.new_empty(B, H, slots, D), t.new_empty(B, slots, dtype=torch.float32),
             t.new_empty(B, slots, dtype=torch.float32))
+
+
+@torch.library.custom_op("gpa::merge_order", mutates_args=())
+def merge_order(cell: Optional[torch.Tensor], frames: int, w: int, h: int, sx: int, sy: int,
+                num_special: int, device: torch.device) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Destination mask (-1 / 0) and token order (destinations, then sources,
+    each by position) of frames x (num_special + w*h) tokens, both int64; cell
+    [frames-1, h//sy, w//sx] int64 is each window's drawn cell, None to draw
+    no patch."""
+    n = frames * (w * h + num_special)
+    mask = torch.empty(n, device=device, dtype=torch.int64)
+    order = torch.empty(n, device=device, dtype=torch.int64)
+    dev = _require_gpu(mask)
+    if cell is not None:
+        _require_gpu(mask, cell)
+        if cell.dtype != torch.int64 or cell.shape != (max(frames - 1, 0), h // sy, w // sx):
+            raise ValueError(f"gpa::merge_order: cell must be int64 [{frames - 1}, {h // sy}, "
+                             f"{w // sx}], got {cell.dtype} {tuple(cell.shape)}")
+        cell = cell.contiguous()
+    with torch.cuda.device(dev):
+        rc = lib().gpa_merge_order(
+            None if cell is None or cell.numel() == 0 else cell.data_ptr(), frames, w, h, sx, sy,
+            num_special, mask.data_ptr(), order.data_ptr(), _stream(dev))
+    _check(rc, "gpa::merge_order")
+    return mask, order
+
+
+@merge_order.register_fake
+def _merge_order_fake(cell, frames, w, h, sx, sy, num_special, device):
+    n = frames * (w * h + num_special)
+    return (torch.empty(n, device=device, dtype=torch.int64),
+            torch.empty(n, device=device, dtype=torch.int64))
+
+
+@torch.library.custom_op("gpa::merge_plan", mutates_args=())
+def merge_plan(node_max: torch.Tensor, node_idx: torch.Tensor, order: torch.Tensor, num_dst: int,
+               r: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor,
+                                torch.Tensor, torch.Tensor, torch.Tensor]:
+    """The merge's index lists from node_max / node_idx [B, num_src] and the
+    token order [num_dst + num_src]: edge [B, num_src], dst_slot [B, r],
+    unm_abs [B, num_src - r], src_abs [B, r], size [B, slots] fp32, offsets
+    [B*slots + 1] and tokens [B*N] (slots: kept sources, then destinations)."""
+    dev = _require_gpu(node_max, node_idx, order)
+    B, ns = node_max.shape
+    N = order.shape[0]
+    if node_max.dtype not in _DTYPE_CODES or node_idx.dtype != torch.int64 \
+            or order.dtype != torch.int64 or node_idx.shape != node_max.shape \
+            or num_dst + ns != N or not 0 <= r <= ns:
+        raise ValueError(f"gpa::merge_plan: node_max {node_max.dtype} {tuple(node_max.shape)}, "
+                         f"node_idx {node_idx.dtype} {tuple(node_idx.shape)}, order {order.dtype} "
+                         f"{tuple(order.shape)}, num_dst {num_dst}, r {r}")
+    node_max, node_idx, order = node_max.contiguous(), node_idx.contiguous(), order.contiguous()
+    slots = ns - r + num_dst
+    new = lambda *shape, dtype=torch.int64: torch.empty(*shape, device=dev, dtype=dtype)  # noqa: E731
+    edge, dst_slot, unm_abs, src_abs = new(B, ns), new(B, r), new(B, ns - r), new(B, r)
+    size, offsets, tokens = new(B, slots, dtype=torch.float32), new(B * slots + 1), new(B * N)
+    if B == 0:
+        return edge, dst_slot, unm_abs, src_abs, size, offsets.zero_(), tokens
+    L = lib()
+    ws_bytes = L.gpa_merge_plan_workspace_bytes(B, ns)
+    ws = new(ws_bytes, dtype=torch.uint8) if ws_bytes else None
+    with torch.cuda.device(dev):
+        rc = L.gpa_merge_plan(
+            node_max.data_ptr(), _DTYPE_CODES[node_max.dtype], node_idx.data_ptr(), order.data_ptr(),
+            B, N, num_dst, r, edge.data_ptr(), dst_slot.data_ptr(), unm_abs.data_ptr(),
+            src_abs.data_ptr(), size.data_ptr(), offsets.data_ptr(), tokens.data_ptr(),
+            ws.data_ptr() if ws is not None else None, ws_bytes, _stream(dev))
+    _check(rc, "gpa::merge_plan")
+    return edge, dst_slot, unm_abs, src_abs, size, offsets, tokens
+
+
+@merge_plan.register_fake
+def _merge_plan_fake(node_max, node_idx, order, num_dst, r):
+    B, ns = node_max.shape
+    slots = ns - r + num_dst
+    e = lambda *shape: node_max.new_empty(shape, dtype=torch.int64)  # noqa: E731
+    return (e(B, ns), e(B, r), e(B, ns - r), e(B, r),
+            node_max.new_empty((B, slots), dtype=torch.float32), e(B * slots + 1),
+            e(B * order.shape[0]))
 
 
 @torch.library.custom_op("gpa::lse_combine", mutates_args=())

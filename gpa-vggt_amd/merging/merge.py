@@ -16,8 +16,10 @@ On the GPU the reference's own calls (`reshape(1, -1, 1).argsort(dim=1)`
 and `argsort(dim=-1, descending=True)`, torch's default sort) give exactly
 these orders, for masks of 1 to 200 frames and node_max rows of 1,045 to
 207,955 entries with tied values (tests/test_gpu_sort_order.py), so the
-stable sorts change no result while making the order a documented property.
-`merge.index` exposes the index tensors for inspection.
+stable orders change no result while making the order a documented property.
+The mask, both orders and the slot lists come from two gfx950 ops
+(`gpa::merge_order`, `gpa::merge_plan`).  `merge.index` exposes the index
+tensors for inspection.
 
 Under bf16 or fp16 autocast (the model's and the evaluation stack's
 cases), or on a bf16 metric, the metric projection, normalisation, dst/src
@@ -66,6 +68,14 @@ def num_dst_tokens(num_imgs: int, w: int, h: int, sx: int, sy: int, num_special:
     return tpi + (num_imgs - 1) * per_frame
 
 
+def window_cells(num_imgs: int, w: int, h: int, sx: int, sy: int,
+                 generator: Optional[torch.Generator], device: torch.device) -> torch.Tensor:
+    """[num_imgs-1, h//sy, w//sx] int64: the cell (row * sx + column) drawn in
+    every window of the frames past the first (reference :105-118)."""
+    return torch.randint(sy * sx, size=(num_imgs - 1, h // sy, w // sx), device=device,
+                         generator=generator)
+
+
 def dst_mask(num_imgs: int, w: int, h: int, sx: int, sy: int, num_special: int,
              no_rand: bool, generator: Optional[torch.Generator],
              device: torch.device) -> torch.Tensor:
@@ -92,8 +102,7 @@ def dst_mask(num_imgs: int, w: int, h: int, sx: int, sy: int, num_special: int,
     if no_rand:
         return mask
     hsy, wsx = h // sy, w // sx
-    cell = torch.randint(sy * sx, size=(num_imgs - 1, hsy, wsx), device=device,
-                         generator=generator)
+    cell = window_cells(num_imgs, w, h, sx, sy, generator, device)
     row_len = wsx * sx
     ys = torch.arange(hsy, device=device).view(1, hsy, 1) * sy + cell // sx
     xs = torch.arange(wsx, device=device).view(1, 1, wsx) * sx + cell % sx
@@ -205,12 +214,13 @@ def token_merge_bipartite2d(
     dev = metric.device
 
     with torch.no_grad():
-        mask = dst_mask(num_imgs, w, h, sx, sy, num_special, no_rand, generator, dev)
         num_dst = num_dst_tokens(num_imgs, w, h, sx, sy, num_special, no_rand)
-        order = torch.argsort(mask, stable=True)  # dst positions first, then src
-        b_pos = order[:num_dst]
-        a_pos = order[num_dst:]
         num_src = N - num_dst
+        cell = None if no_rand or num_imgs <= 1 else window_cells(num_imgs, w, h, sx, sy,
+                                                                  generator, dev)
+        mask, order = torch.ops.gpa.merge_order(cell, num_imgs, w, h, sx, sy, num_special, dev)
+        b_pos = order[:num_dst]                   # dst positions first, then src
+        a_pos = order[num_dst:]
 
         front = _front_end_mode(metric, C, metric_dim)
         if front is not None:
@@ -244,34 +254,14 @@ def token_merge_bipartite2d(
         else:
             node_max = torch.empty(B, 0, device=dev, dtype=max_dtype)
             node_idx = torch.empty(B, 0, device=dev, dtype=torch.int64)
-        edge = torch.argsort(node_max, dim=-1, descending=True, stable=True)
-        src_rank = edge[:, :r]          # merged source rows (rows of `a`)
-        unm_rank = edge[:, r:]          # kept source rows
-        dst_slot = torch.gather(node_idx, 1, src_rank)        # [B, r] dst slot per merged row
-        unm_abs = a_pos[unm_rank]                             # [B, unm_len] token positions
-        src_abs = a_pos[src_rank]                             # [B, r]
-        unm_len = unm_rank.shape[1]
-
-        size = torch.ones(B, unm_len + num_dst, device=dev, dtype=torch.float32)
-        size[:, unm_len:].scatter_add_(1, dst_slot, torch.ones(B, r, device=dev,
-                                                                dtype=torch.float32))
-
-        # Token list of every output slot, for the deterministic merge
-        # kernel: slot i < unm_len holds kept source token unm_abs[i]; dst
-        # slot unm_len + j holds dst token b_pos[j] first, then the source
-        # tokens merged into it in increasing position.  Every input token
-        # appears exactly once, so each batch element lists N tokens.
+        # Slot i < unm_len holds kept source token unm_abs[i]; dst slot
+        # unm_len + j holds dst token b_pos[j] first, then the source tokens
+        # merged into it in increasing position.  Every input token appears
+        # exactly once, so each batch element lists N tokens.
+        edge, dst_slot, unm_abs, src_abs, size, csr_offsets, csr_tokens = torch.ops.gpa.merge_plan(
+            node_max, node_idx, order, num_dst, r)
+        unm_len = num_src - r
         slots = unm_len + num_dst
-        key = torch.cat([torch.arange(unm_len, device=dev).expand(B, unm_len),
-                         (unm_len + torch.arange(num_dst, device=dev)).expand(B, num_dst),
-                         unm_len + dst_slot], dim=1)
-        tok = torch.cat([unm_abs, b_pos.expand(B, num_dst), src_abs], dim=1)
-        sub = torch.cat([torch.zeros(B, unm_len + num_dst, device=dev, dtype=torch.int64),
-                         src_abs + 1], dim=1)      # the slot's own token sorts first
-        order = torch.argsort(key * (N + 1) + sub, dim=1)
-        csr_tokens = torch.gather(tok, 1, order).reshape(-1)
-        csr_offsets = torch.zeros(B * slots + 1, device=dev, dtype=torch.int64)
-        csr_offsets[1:] = torch.cumsum(size.reshape(-1).to(torch.int64), 0)
 
     def kernel_merge(t: torch.Tensor, mode: str) -> Optional[torch.Tensor]:
         """The deterministic gfx950 merge for sum / mean of fp32, bf16 and

@@ -1,7 +1,7 @@
 /*
  * gpa_mi355x.h — C ABI of the MI355X (gfx950) GPA-VGGT merging hot path.
  *
- * Eight entry points (two of them with an fp16 twin, the attention also
+ * Ten entry points (two of them with an fp16 twin, the attention also
  * with an allocation-free variant) sit behind this boundary:
  *
  *   gpa_sim_argmax_bf16   — fused cosine-similarity row max / argmax between
@@ -14,6 +14,9 @@
  *   gpa_merge_heads       — deterministic segmented mean/sum of token rows,
  *                           the K/V merge (replaces the scatter_reduce_ of
  *                           merging/merge.py:234-250).
+ *   gpa_merge_order, gpa_merge_plan — the merge's bookkeeping: destination
+ *                           mask, token and merge orders, slot token lists
+ *                           (replaces merging/merge.py:85-165, 196-217).
  *   gpa_lse_combine_bf16  — merge of two partial attentions by their log2
  *                           LSE (replaces vggt/layers/attention.py:166-176).
  *   gpa_qk_norm_rope_bf16 (and _f16) — qk LayerNorm + 2D RoPE + cast of a block's
@@ -55,7 +58,7 @@
 extern "C" {
 #endif
 
-#define GPA_ABI_VERSION 15
+#define GPA_ABI_VERSION 16
 
 enum {
   GPA_OK = 0,
@@ -231,6 +234,44 @@ int gpa_merge_heads(const void* t, int dtype, void* out,
                     int64_t t_sb, int64_t t_sh, int64_t t_sn,
                     int64_t o_sb, int64_t o_sh, int64_t o_sn,
                     int mode, float* size_out, float* log_size_out, void* stream);
+
+/*
+ * Destination mask and token order of the bipartite merge
+ * (merging/merge.py:85-165) over `frames` frames of num_special + w*h tokens:
+ * every token of frame 0 and the special tokens of every frame are
+ * destinations, and in each frame past the first one cell per sy x sx window:
+ *   cell [frames-1, h/sy, w/sx] int64, the drawn cell (row * sx + column) of
+ *        each window, or NULL to mark no patch
+ *   mask [frames * (w*h + num_special)] int64: -1 destination, 0 source
+ *   order, same length: the positions of the destinations, then those of the
+ *        sources, each increasing
+ */
+int gpa_merge_order(const int64_t* cell, int64_t frames, int64_t w, int64_t h,
+                    int64_t sx, int64_t sy, int64_t num_special,
+                    int64_t* mask, int64_t* order, void* stream);
+
+/* Bytes of device workspace gpa_merge_plan needs (16-byte aligned). */
+size_t gpa_merge_plan_workspace_bytes(int64_t B, int64_t num_src);
+
+/*
+ * The merge itself as index lists (merging/merge.py:196-217), per batch
+ * element, from the similarity's row maxima over num_src = N - num_dst sources:
+ *   node_max [B, num_src] (max_dtype elements), node_idx [B, num_src] int64,
+ *   order [N] int64 as gpa_merge_order writes it; r sources are merged
+ *   edge [B, num_src]: source rows by descending node_max (NaN first), ties by
+ *        increasing row
+ *   dst_slot [B, r], src_abs [B, r]: destination and token position of
+ *        edge[:r]; unm_abs [B, num_src - r]: token positions of edge[r:]
+ *   size [B, S] fp32, offsets [B*S + 1], tokens [B*N] (S = num_src - r +
+ *        num_dst): the slot lists gpa_merge_heads takes, slots [kept sources |
+ *        destinations], each slot's own token first, then its merged sources
+ *        by increasing position
+ */
+int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t* node_idx,
+                   const int64_t* order, int64_t B, int64_t N, int64_t num_dst, int64_t r,
+                   int64_t* edge, int64_t* dst_slot, int64_t* unm_abs, int64_t* src_abs,
+                   float* size, int64_t* offsets, int64_t* tokens,
+                   void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Merge of two attentions over a partition of the keys by their log2 LSE,

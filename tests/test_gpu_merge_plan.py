@@ -1,0 +1,76 @@
+"""The merge's bookkeeping kernels (gpa::merge_order, gpa::merge_plan) against
+torch's stable sorts: exact, every output.  Row counts sit at the edges of the
+one-workgroup path (8,192 rows) and of the radix sort's blocks (4,096 rows);
+maxima with ties, NaN, both zeros and infinities; all rows of a batch element
+in one slot; destination counts of one to three key bytes."""
+import pytest
+import torch
+
+from merging import _native  # noqa: F401  (registers the ops)
+from merging.merge import dst_mask, num_dst_tokens, window_cells
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("frames,w,h,sx,sy,ns,no_rand", [
+    (1, 37, 37, 2, 2, 5, False), (3, 37, 37, 2, 2, 5, False), (9, 37, 28, 2, 3, 5, False),
+    (4, 5, 7, 3, 2, 0, False), (4, 6, 6, 2, 2, 5, True), (2, 3, 3, 4, 4, 1, False),
+    (2, 45, 45, 1, 1, 7, False)])
+def test_order_and_mask(dev, frames, w, h, sx, sy, ns, no_rand):
+    def gen():
+        return torch.Generator(device=dev).manual_seed(frames)
+
+    mask = dst_mask(frames, w, h, sx, sy, ns, no_rand, gen(), dev)
+    cell = None if no_rand or frames == 1 else window_cells(frames, w, h, sx, sy, gen(), dev)
+    got_mask, got = torch.ops.gpa.merge_order(cell, frames, w, h, sx, sy, ns, dev)
+    assert torch.equal(got_mask, mask)
+    assert torch.equal(got, torch.argsort(mask, stable=True))
+    assert int((mask == -1).sum()) == num_dst_tokens(frames, w, h, sx, sy, ns, no_rand)
+
+
+def _expected(node_max, node_idx, order, num_dst, r):
+    """The same lists from torch's stable sorts, on the CPU."""
+    B, ns = node_max.shape
+    N = num_dst + ns
+    b_pos, a_pos = order[:num_dst], order[num_dst:]
+    edge = torch.argsort(node_max.float(), dim=-1, descending=True, stable=True)
+    dst_slot = torch.gather(node_idx, 1, edge[:, :r])
+    unm_abs, src_abs = a_pos[edge[:, r:]], a_pos[edge[:, :r]]
+    unm = ns - r
+    size = torch.ones(B, unm + num_dst)
+    size[:, unm:].scatter_add_(1, dst_slot, torch.ones(B, r))
+    key = torch.cat([torch.arange(unm + num_dst).expand(B, -1), unm + dst_slot], 1)
+    tok = torch.cat([unm_abs, b_pos.expand(B, num_dst), src_abs], 1)
+    sub = torch.cat([torch.zeros(B, unm + num_dst, dtype=torch.int64), src_abs + 1], 1)
+    tokens = torch.gather(tok, 1, torch.argsort(key * (N + 1) + sub, dim=1)).reshape(-1)
+    offsets = torch.zeros(B * (unm + num_dst) + 1, dtype=torch.int64)
+    offsets[1:] = torch.cumsum(size.reshape(-1).to(torch.int64), 0)
+    return edge, dst_slot, unm_abs, src_abs, size, offsets, tokens
+
+
+@pytest.mark.parametrize("ns", [0, 1, 64, 1023, 1045, 8191, 8192, 8193, 12288, 20481])
+@pytest.mark.parametrize("num_dst,share,dtype,kind", [
+    (1, 1.0, torch.float32, "plain"), (255, 0.2, torch.float32, "ties"),
+    (256, 1.0, torch.bfloat16, "special"), (300, 0.0, torch.float16, "ties"),
+    (70_000, 0.5, torch.float32, "special")])
+def test_plan(dev, ns, num_dst, share, dtype, kind):
+    g = torch.Generator().manual_seed(ns + num_dst)
+    B = 1 if ns == 1045 else 2
+    node_max = torch.randn(B, ns, generator=g)
+    if kind == "ties":
+        node_max = (node_max * 4).round() / 4
+    elif kind == "special" and ns > 0:
+        pool = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), 1.0, -1.0])
+        pick = torch.randint(0, 14, (B, ns), generator=g)
+        node_max = torch.where(pick < 7, pool[pick.clamp_max(6)], node_max)
+    node_max = node_max.to(dtype)
+    node_idx = torch.randint(0, num_dst, (B, ns), generator=g)
+    node_idx[B - 1, ns // 3:] = num_dst - 1                 # most rows in one slot
+    order = torch.randperm(num_dst + ns, generator=g)
+    order = torch.cat([order[:num_dst].sort().values, order[num_dst:].sort().values])
+    r = int(ns * share)
+    want = _expected(node_max, node_idx, order, num_dst, r)
+    got = torch.ops.gpa.merge_plan(node_max.to(dev), node_idx.to(dev), order.to(dev), num_dst, r)
+    for name, x, y in zip(("edge", "dst_slot", "unm_abs", "src_abs", "size", "offsets", "tokens"),
+                          got, want):
+        assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
