@@ -51,6 +51,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from merging import _native
 from merging.fused_attention import attention_keybias, combine_by_lse
 from merging.merge import token_merge_bipartite2d
 
@@ -241,7 +242,7 @@ class GpaAttention(nn.Module):
                                  "projection (run the model under bf16 or fp16 autocast)")
             ln_w = torch.stack((self.q_norm.weight, self.k_norm.weight))
             ln_b = torch.stack((self.q_norm.bias, self.k_norm.bias))
-            q, k = torch.ops.gpa.qk_norm_rope(
+            q, k = _native.qk_norm_rope(
                 qkv, ln_w, ln_b, self.q_norm.eps, None if rope is None else rope.pos,
                 None if rope is None else rope.cs, H, False, k_f32)
             return q, k, v
@@ -354,7 +355,7 @@ def pool_shared_set(k: torch.Tensor, v: torch.Tensor, frames: int, pts: int, gri
     fp32, assign [B, H, S, grid_h*grid_w] or an empty tensor)."""
     if (grid_h * grid_w <= POOL_KERNEL_MAX_PATCHES and k.shape[-1] == 64
             and k.dtype in (torch.bfloat16, torch.float16)):
-        return torch.ops.gpa.pool_shared(k, v, frames, pts, grid_h, grid_w, kp, want_assign)
+        return _native.pool_shared(k, v, frames, pts, grid_h, grid_w, kp, want_assign)
     B, H, N, D = k.shape
     P = N // frames
     pk, pv, size, assign = pool_shared_torch(k.view(B, H, frames, P, D),
@@ -426,7 +427,7 @@ class Block(nn.Module):
             # block.py:84-96 with the elementwise steps fused: LayerNorm 1 to
             # the 16-bit format; x + ls1(attn) with LayerNorm 2 in one pass;
             # x + ls2(mlp).
-            rl = torch.ops.gpa.residual_layernorm
+            rl = _native.residual_layernorm
             _, ln1 = rl(x, None, None, self.norm1.weight, self.norm1.bias, self.norm1.eps, False)
             a = self.attn(ln1, rope, global_merging)
             h, ln2 = rl(x, a, self.ls1.gamma, self.norm2.weight, self.norm2.bias,

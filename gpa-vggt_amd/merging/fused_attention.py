@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _native  # noqa: F401  (registers torch.ops.gpa.*)
+from . import _native
 
 __all__ = ["attention_keybias", "combine_by_lse", "LOG2E"]
 
@@ -51,7 +51,7 @@ def attention_keybias(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         raise ValueError("attention_keybias expects [B, H, T, D] q/k/v")
     v = v.to(q.dtype)
     k = k.to(q.dtype)
-    o, lse = torch.ops.gpa.attn_keybias(q, k, v, bias, float(sm_scale), bool(return_lse))
+    o, lse = _native.attn_keybias(q, k, v, bias, float(sm_scale), bool(return_lse))
     return (o, lse) if return_lse else o
 
 
@@ -68,4 +68,4 @@ def combine_by_lse(out_a: torch.Tensor, lse_a: torch.Tensor, out_b: torch.Tensor
     The weights and the sum are fp32 (the reference rounds the weights to the
     activation dtype first).
     """
-    return torch.ops.gpa.lse_combine(out_a, lse_a, out_b, lse_b, int(frames))
+    return _native.lse_combine(out_a, lse_a, out_b, lse_b, int(frames))

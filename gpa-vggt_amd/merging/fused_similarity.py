@@ -54,5 +54,5 @@ def fused_similarity_argmax(a: torch.Tensor, b: torch.Tensor):
         b = F.pad(b, (0, pad))
     # The kernel writes the max in a's 16-bit dtype itself when that is the
     # output dtype (fp32 inputs keep the fp32 max).
-    node_max, node_idx = torch.ops.gpa.sim_argmax(a, b, out_dtype == a.dtype)
+    node_max, node_idx = _native.sim_argmax(a, b, out_dtype == a.dtype)
     return node_max.to(out_dtype), node_idx

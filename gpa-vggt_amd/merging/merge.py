@@ -218,7 +218,7 @@ def token_merge_bipartite2d(
         num_src = N - num_dst
         cell = None if no_rand or num_imgs <= 1 else window_cells(num_imgs, w, h, sx, sy,
                                                                   generator, dev)
-        mask, order = torch.ops.gpa.merge_order(cell, num_imgs, w, h, sx, sy, num_special, dev)
+        mask, order = _native.merge_order(cell, num_imgs, w, h, sx, sy, num_special, dev)
         b_pos = order[:num_dst]                   # dst positions first, then src
         a_pos = order[num_dst:]
 
@@ -247,7 +247,7 @@ def token_merge_bipartite2d(
 
         r = min(num_src, r)
         if num_src > 0 and front is not None:
-            node_max, node_idx = torch.ops.gpa.sim_argmax(a, b)     # fp32 row max
+            node_max, node_idx = _native.sim_argmax(a, b)     # fp32 row max
             node_max = node_max.to(max_dtype)
         elif num_src > 0:
             node_max, node_idx = fused_similarity_argmax(a, b)
@@ -258,7 +258,7 @@ def token_merge_bipartite2d(
         # unm_len + j holds dst token b_pos[j] first, then the source tokens
         # merged into it in increasing position.  Every input token appears
         # exactly once, so each batch element lists N tokens.
-        edge, dst_slot, unm_abs, src_abs, size, csr_offsets, csr_tokens = torch.ops.gpa.merge_plan(
+        edge, dst_slot, unm_abs, src_abs, size, csr_offsets, csr_tokens = _native.merge_plan(
             node_max, node_idx, order, num_dst, r)
         unm_len = num_src - r
         slots = unm_len + num_dst
