@@ -140,6 +140,19 @@ struct AttnArgs {
   int no_bound;                           // records without key maxima: no score bound
 };
 
+// Another attention of the same queries over further keys, joined by LSE,
+// contiguous and frame-major: o [B * M / P, H, P, 64], lse [B * M / P, H, P].
+struct JoinArgs {
+  const uint16_t* o;
+  const float* lse;
+  int P;
+};
+
+struct AttnJoinArgs {
+  AttnArgs a;
+  JoinArgs join;
+};
+
 struct RecArgs {
   const uint16_t* k;
   const void* bias;
@@ -407,8 +420,8 @@ struct alignas(16) MainTile {
   float rec[64];
 };
 
-template <bool F16>
-__global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
+template <bool F16, bool JOIN>
+__device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
   __shared__ MainTile ring0, ring1, ring2, ring3, ring4;
   __shared__ float rec_sink[64];
   __shared__ uint32_t wg_fail[kWaves];   // per wave: its tile-0 offset overflowed
@@ -440,9 +453,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
   // The output bases, formed here so that only two pointers (not five
   // 64-bit strides) stay live in SGPRs until the epilogue.
   uint16_t* O = p.o + b * p.o_sb + h * p.o_sh;
-  float* LSE = p.lse ? p.lse + b * p.lse_sb + h * p.lse_sh : nullptr;
+  float* LSE = !JOIN && p.lse ? p.lse + b * p.lse_sb + h * p.lse_sh : nullptr;
   const int o_sm = (int)p.o_sm;
-  asm volatile("" : "+s"(O), "+s"(LSE));
+  if constexpr (JOIN) asm volatile("" : "+s"(O));
+  else asm volatile("" : "+s"(O), "+s"(LSE));
 
   // Q^T as the B-operand of S^T = K . Q^T: in block j the lane supplies
   // query q_base + 32 j, features 16*ks + 8*hi .. +8.  Only the loads here:
@@ -883,30 +897,87 @@ __global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
   // second pass, already saw every wave's last ring read.)
   MainTile& slot_w = wave == 0 ? ring0 : wave == 1 ? ring1 : wave == 2 ? ring2 : ring3;
   uint16_t* const stage = reinterpret_cast<uint16_t*>(&slot_w);
+  const int64_t row0 = (int64_t)qb * kQPerWG + wave * kQPerWave;
+  const int ch = lane & 7;
+  constexpr int kRowSets = kQPerWave / 8;
+  JoinArgs join{};
+  uint64_t join_row0 = 0;
+  uint32_t frame_rows = 0;
+  // Token n is row n % P of frame n / P; a frame is H * P rows, of which this
+  // head's start at join_row0 in frame 0.
+  auto join_row = [&](int64_t row) {
+    const uint32_t s = (uint32_t)row / (uint32_t)join.P;
+    return join_row0 + (uint64_t)s * frame_rows + ((uint32_t)row - s * (uint32_t)join.P);
+  };
+  if constexpr (JOIN) {
+    // Read from the argument segment only here (the empty asm keeps the loads
+    // below the loop: held from the start they spill 9 SGPRs).
+    typedef __attribute__((address_space(4))) const AttnJoinArgs* Args;
+    Args args = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    join.o = args->join.o;
+    join.lse = args->join.lse;
+    join.P = args->join.P;
+    const uint32_t heads = (uint32_t)args->a.H, jb = (uint32_t)bh / heads, jh = (uint32_t)bh % heads;
+    frame_rows = heads * (uint32_t)join.P;
+    join_row0 = ((uint64_t)jb * ((uint32_t)p.M / (uint32_t)join.P) * heads + jh) * (uint32_t)join.P;
+    // The other attention's rows take the way of the stores below backwards:
+    // whole rows into the stage, from where each lane reads the features of
+    // its query where it will write the joined ones.
+    u32x4 other[kRowSets];
+#pragma unroll
+    for (int i = 0; i < kRowSets; ++i) {
+      const int64_t row = row0 + 8 * i + (lane >> 3);
+      other[i] = row < p.M ? *reinterpret_cast<const u32x4*>(join.o + join_row(row) * kHD + ch * 8)
+                           : u32x4{};
+    }
+#pragma unroll
+    for (int i = 0; i < kRowSets; ++i) {
+      const int r = 8 * i + (lane >> 3);
+      *reinterpret_cast<u32x4*>(&stage[r * kHD + ((ch ^ (r & 7)) << 3)]) = other[i];
+    }
+  }
 #pragma unroll
   for (int j = 0; j < kBlk; ++j) {
     const int r = 32 * j + l32;
+    const int64_t row = q_base + 32 * j;
     const float l_tot = sum_halves(l_acc[j][0]);
-    const float inv = 1.0f / l_tot;
+    float inv = 1.0f / l_tot, w_other = 0.f;
+    if constexpr (JOIN) {
+      // Both halves in fp32; weights 2^(lse - max) over their sum.
+      const float la = row < p.M ? join.lse[join_row(row)] : 0.f;
+      const float lb = m_off[j] + __log2f(l_tot), top = fmaxf(la, lb);
+      const float wa = __builtin_amdgcn_exp2f(la - top), wb = __builtin_amdgcn_exp2f(lb - top);
+      const float norm = 1.0f / (wa + wb);
+      w_other = wa * norm;
+      inv *= wb * norm;
+    }
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int cw = db * 4 + g;
-        const bf16x4 ov = {f32_to_half<F16>(o_acc[j][db][4 * g + 0] * inv),
-                           f32_to_half<F16>(o_acc[j][db][4 * g + 1] * inv),
-                           f32_to_half<F16>(o_acc[j][db][4 * g + 2] * inv),
-                           f32_to_half<F16>(o_acc[j][db][4 * g + 3] * inv)};
-        *reinterpret_cast<bf16x4*>(&stage[r * kHD + ((cw ^ (r & 7)) << 3) + 4 * hi]) = ov;
+        bf16x4* const at =
+            reinterpret_cast<bf16x4*>(&stage[r * kHD + ((cw ^ (r & 7)) << 3) + 4 * hi]);
+        bf16x4 ov;
+        if constexpr (JOIN) {
+          const bf16x4 x = *at;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            ov[e] = f32_to_half<F16>(__builtin_fmaf(half_to_f32<F16>(x[e]), w_other,
+                                                    o_acc[j][db][4 * g + e] * inv));
+        } else {
+          ov = bf16x4{f32_to_half<F16>(o_acc[j][db][4 * g + 0] * inv),
+                      f32_to_half<F16>(o_acc[j][db][4 * g + 1] * inv),
+                      f32_to_half<F16>(o_acc[j][db][4 * g + 2] * inv),
+                      f32_to_half<F16>(o_acc[j][db][4 * g + 3] * inv)};
+        }
+        *at = ov;
       }
-    const int64_t row = q_base + 32 * j;
-    if (LSE && hi == 0 && row < p.M) LSE[row] = m_off[j] + __log2f(l_tot);
+    if (!JOIN && LSE && hi == 0 && row < p.M) LSE[row] = m_off[j] + __log2f(l_tot);
   }
   // All eight row reads first, then the stores (read-wait-store in turn
   // serialised eight LDS round trips).
-  const int64_t row0 = (int64_t)qb * kQPerWG + wave * kQPerWave;
-  const int ch = lane & 7;
-  constexpr int kRowSets = kQPerWave / 8;
   u32x4 ov16[kRowSets];
 #pragma unroll
   for (int i = 0; i < kRowSets; ++i) {
@@ -930,6 +1001,21 @@ __global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
       }
     }
   }
+}
+
+template <bool F16>
+__global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
+  attn_main_body<F16, false>(p);
+}
+
+// The second attention of a split key set, joined with the first in its
+// epilogue: one read of the first's rows instead of writing this one's,
+// reading both back and another launch (26 us at 16 frames, 21,984 queries,
+// 16 heads; with the shared set written by one kernel too, the block went
+// from 569 to 524 us).
+template <bool F16>
+__global__ __launch_bounds__(kThreads, 2) void attn_join_kernel(AttnJoinArgs p) {
+  attn_main_body<F16, true>(p.a);
 }
 
 // Workspace: one row of ntiles tile records per (batch, head), then
@@ -966,7 +1052,8 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
                      int64_t N, int64_t D, int64_t q_sb, int64_t q_sh, int64_t q_sm, int64_t k_sb,
                      int64_t k_sh, int64_t k_sn, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                      int64_t o_sb, int64_t o_sh, int64_t o_sm, int64_t lse_sb, int64_t lse_sh,
-                     void* workspace, size_t workspace_bytes, float sm_scale, void* stream) {
+                     void* workspace, size_t workspace_bytes, float sm_scale, void* stream,
+                     const JoinArgs* join = nullptr) {
   gpa_clear_error();
   if (B < 0 || H < 0 || M < 0 || N < 0 || D < 0) {
     gpa_set_error("%s: negative size", fn);
@@ -981,8 +1068,14 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
     gpa_set_error("%s: head_dim %lld unsupported (16, 32, 64, 128 or 256)", fn, (long long)D);
     return GPA_E_UNSUPPORTED;
   }
-  if (!q || !k || !v || !o) {
+  if (!q || !k || !v || !o || (join && (!join->o || !join->lse))) {
     gpa_set_error("%s: null tensor pointer", fn);
+    return GPA_E_INVALID;
+  }
+  if (join && (D != kHD || join->P <= 0 || M % join->P != 0 || M > 0x7fffffff ||
+               H * join->P > 0x7fffffff || (uintptr_t)join->o % 16)) {
+    gpa_set_error("%s: the joined attention takes head dim 64, M=%lld a multiple of P=%d and "
+                  "16-byte aligned rows", fn, (long long)M, join->P);
     return GPA_E_INVALID;
   }
   if (bias_kind != GPA_BIAS_NONE && bias_kind != GPA_BIAS_F32 && bias_kind != GPA_BIAS_BF16 &&
@@ -1161,7 +1254,10 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
   p.no_bound = no_bound ? 1 : 0;
 
   const dim3 grid((unsigned)gx, (unsigned)(B * H)), block(kThreads);
-  hipLaunchKernelGGL(attn_main_kernel<F16>, grid, block, 0, s, p);
+  if (join)
+    hipLaunchKernelGGL(attn_join_kernel<F16>, grid, block, 0, s, AttnJoinArgs{p, *join});
+  else
+    hipLaunchKernelGGL(attn_main_kernel<F16>, grid, block, 0, s, p);
   e = hipGetLastError();
   if (e != hipSuccess) {
     gpa_set_error("%s: launch failed: %s", fn, hipGetErrorString(e));
@@ -1200,6 +1296,29 @@ extern "C" int gpa_attn_keybias_f16(const void* q, const void* k, const void* v,
                                 bias_sh, bias_sn, o, lse, B, H, M, N, D, q_sb, q_sh, q_sm, k_sb,
                                 k_sh, k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sm, lse_sb, lse_sh,
                                 workspace, workspace_bytes, sm_scale, stream);
+}
+
+extern "C" int gpa_attn_keybias_join(
+    int dtype, const void* q, const void* k, const void* v, const void* bias, int bias_kind,
+    int64_t bias_sb, int64_t bias_sh, int64_t bias_sn, const void* other_o, const float* other_lse,
+    int64_t P, void* o, int64_t B, int64_t H, int64_t M, int64_t N, int64_t D, int64_t q_sb, int64_t q_sh, int64_t q_sm, int64_t k_sb, int64_t k_sh,
+    int64_t k_sn, int64_t v_sb, int64_t v_sh, int64_t v_sn, int64_t o_sb, int64_t o_sh,
+    int64_t o_sm, void* workspace, size_t workspace_bytes, float sm_scale, void* stream) {
+  static const char* fn = "gpa_attn_keybias_join";
+  const JoinArgs join{(const uint16_t*)other_o, other_lse, P > 0 && P <= 0x7fffffff ? (int)P : 0};
+  if (dtype == GPA_DTYPE_BF16)
+    return attn_keybias_run<false>(fn, q, k, v, bias, bias_kind, bias_sb, bias_sh, bias_sn, o,
+                                   nullptr, B, H, M, N, D, q_sb, q_sh, q_sm, k_sb, k_sh, k_sn,
+                                   v_sb, v_sh, v_sn, o_sb, o_sh, o_sm, 0, 0, workspace,
+                                   workspace_bytes, sm_scale, stream, &join);
+  if (dtype == GPA_DTYPE_F16)
+    return attn_keybias_run<true>(fn, q, k, v, bias, bias_kind, bias_sb, bias_sh, bias_sn, o,
+                                  nullptr, B, H, M, N, D, q_sb, q_sh, q_sm, k_sb, k_sh, k_sn,
+                                  v_sb, v_sh, v_sn, o_sb, o_sh, o_sm, 0, 0, workspace,
+                                  workspace_bytes, sm_scale, stream, &join);
+  gpa_clear_error();
+  gpa_set_error("%s: unknown dtype %d", fn, dtype);
+  return GPA_E_INVALID;
 }
 
 // ---------------------------------------------------------------------------

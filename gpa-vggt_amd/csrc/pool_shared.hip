@@ -59,6 +59,8 @@ struct PoolArgs {
   uint16_t* pv;
   float* size;
   int32_t* assign;   // nullable
+  uint16_t* bias;    // nullable: [B, H, out_bh], with the special tokens' rows (see write_set)
+  int64_t out_bh, out_off;   // pk / pv rows per (batch, head), first pooled row
   int64_t k_sb, k_sh, k_sn, v_sb, v_sh, v_sn;
   int H, S, P, pts, gh, gw, kp, nw, npool;
 };
@@ -76,6 +78,28 @@ __device__ __forceinline__ float round16(float x) { return half_to_f32<F16>(f32_
 // 1.0 in the 16-bit format: the one-hot A operand.
 template <bool F16>
 constexpr uint32_t kOne16 = F16 ? 0x3c00u : 0x3f80u;
+
+// The rest of a frame's part of the shared set (bias given): the special
+// tokens' keys and values in rows s*pts .. of the (batch, head)'s output, and
+// the bias row, 0 there and log(size) at the pooled keys (an empty group
+// gets -inf).  K and V point at the frame's first patch.  As torch operations
+// the concatenations, the zeros, the logs and the conversions were nine
+// launches and ~45 us of a 16-frame block.
+template <bool F16>
+__device__ __forceinline__ void write_set(const PoolArgs& a, int bh, int s, const uint16_t* K,
+                                          const uint16_t* V, int64_t out_row0, const int* count) {
+  const int64_t row0 = bh * a.out_bh + (int64_t)s * a.pts;
+  for (int i = threadIdx.x; i < a.pts * (kPoolD / 8); i += kPoolThreads) {
+    const int r = i / (kPoolD / 8), c = i % (kPoolD / 8) * 8;
+    *reinterpret_cast<u32x4*>(a.pk + (row0 + r) * kPoolD + c) =
+        *reinterpret_cast<const u32x4*>(K + (int64_t)(r - a.pts) * a.k_sn + c);
+    *reinterpret_cast<u32x4*>(a.pv + (row0 + r) * kPoolD + c) =
+        *reinterpret_cast<const u32x4*>(V + (int64_t)(r - a.pts) * a.v_sn + c);
+  }
+  for (int i = threadIdx.x; i < a.pts; i += kPoolThreads) a.bias[row0 + i] = 0;
+  for (int g = threadIdx.x; g < a.npool; g += kPoolThreads)
+    a.bias[out_row0 + g] = __builtin_bit_cast(uint16_t, f32_to_half<F16>(logf((float)count[g])));
+}
 
 // NSB: blocks of 32 seeds (1 or 2), so the accumulators of an absent block
 // take no registers.  One block fits three waves per SIMD without spills
@@ -150,7 +174,8 @@ void pool_shared_kernel(PoolArgs a) {
 
   uint16_t(&st)[32][kStage] = stage[wave];
   const int ntile = (npatch + 31) / 32;        // ntile * 32 <= kMaxPatches
-  const int64_t out_row0 = ((int64_t)bh * a.S + s) * a.npool;   // row of [B, H, S*npool]
+  const int64_t size_row0 = ((int64_t)bh * a.S + s) * a.npool;  // row of [B, H, S*npool]
+  const int64_t out_row0 = bh * a.out_bh + a.out_off + (int64_t)s * a.npool;
 
   // Score a tile's normalised rows against the seeds; the row's seed (lowest
   // on ties) goes to asg, the count and the optional assignment output.
@@ -269,7 +294,8 @@ void pool_shared_kernel(PoolArgs a) {
   };
   sweep(K, a.k_sn, true, PK);
   sweep(Vp, a.v_sn, false, PV);
-  for (int g = tid; g < a.npool; g += kPoolThreads) SZ[out_row0 + g] = (float)count[g];
+  for (int g = tid; g < a.npool; g += kPoolThreads) SZ[size_row0 + g] = (float)count[g];
+  if (a.bias) write_set<F16>(a, bh, s, K, Vp, out_row0, count);
 }
 
 // More than 64 seeds per frame (pool stride <= 4 at grid 37, down to every
@@ -325,7 +351,8 @@ __global__ __launch_bounds__(kPoolThreads, 2) void pool_many_kernel(PoolArgs a) 
   const int nsc = (a.npool + kMaxPool - 1) / kMaxPool;
   const uint16_t* K = a.k + b * a.k_sb + h * a.k_sh + ((int64_t)s * a.P + a.pts) * a.k_sn;
   const uint16_t* Vp = a.v + b * a.v_sb + h * a.v_sh + ((int64_t)s * a.P + a.pts) * a.v_sn;
-  const int64_t out_row0 = ((int64_t)bh * a.S + s) * a.npool;
+  const int64_t size_row0 = ((int64_t)bh * a.S + s) * a.npool;
+  const int64_t out_row0 = bh * a.out_bh + a.out_off + (int64_t)s * a.npool;
   uint16_t* PK = a.pk;
   uint16_t* PV = a.pv;
   float* SZ = a.size;
@@ -657,7 +684,8 @@ __global__ __launch_bounds__(kPoolThreads, 2) void pool_many_kernel(PoolArgs a) 
       if (gs < ge) flush(ge);
     }
   }
-  for (int g = tid; g < a.npool; g += kPoolThreads) SZ[out_row0 + g] = (float)count[g];
+  for (int g = tid; g < a.npool; g += kPoolThreads) SZ[size_row0 + g] = (float)count[g];
+  if (a.bias) write_set<F16>(a, bh, s, K, Vp, out_row0, count);
 }
 
 }  // namespace
@@ -674,7 +702,7 @@ int pool_run(const char* fn, const void* k, const void* v, void* pooled_k, void*
              float* size, int32_t* assign, int64_t B, int64_t H, int64_t S, int64_t P,
              int64_t pts, int64_t grid_h, int64_t grid_w, int64_t kp, int64_t D, int64_t k_sb,
              int64_t k_sh, int64_t k_sn, int64_t v_sb, int64_t v_sh, int64_t v_sn,
-             void* stream) {
+             void* stream, void* bias = nullptr, bool whole_set = false) {
   gpa_clear_error();
   if (B < 0 || H < 0 || S < 0 || P < 0 || pts < 0 || grid_h < 0 || grid_w < 0 || kp <= 0) {
     gpa_set_error("%s: negative size or kp <= 0", fn);
@@ -685,7 +713,7 @@ int pool_run(const char* fn, const void* k, const void* v, void* pooled_k, void*
     return GPA_E_UNSUPPORTED;
   }
   if (B == 0 || H == 0 || S == 0 || grid_h == 0 || grid_w == 0) return GPA_OK;
-  if (!k || !v || !pooled_k || !pooled_v || !size) {
+  if (!k || !v || !pooled_k || !pooled_v || !size || (whole_set && !bias)) {
     gpa_set_error("%s: null pointer", fn);
     return GPA_E_INVALID;
   }
@@ -722,11 +750,14 @@ int pool_run(const char* fn, const void* k, const void* v, void* pooled_k, void*
   a.pv = (uint16_t*)pooled_v;
   a.size = size;
   a.assign = assign;
+  a.bias = (uint16_t*)bias;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
   a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
   a.H = (int)H; a.S = (int)S; a.P = (int)P; a.pts = (int)pts;
   a.gh = (int)grid_h; a.gw = (int)grid_w;
   a.kp = (int)kp; a.nw = (int)nw; a.npool = (int)(nh * nw);
+  a.out_off = whole_set ? S * pts : 0;
+  a.out_bh = a.out_off + S * a.npool;
   if (a.npool > kMaxPool)
     hipLaunchKernelGGL((pool_many_kernel<F16>), dim3((unsigned)groups), dim3(kPoolThreads), 0,
                        (hipStream_t)stream, a);
@@ -761,4 +792,21 @@ extern "C" int gpa_pool_shared_bf16(GPA_POOL_ARGS) {
 
 extern "C" int gpa_pool_shared_f16(GPA_POOL_ARGS) {
   return pool_run<true>("gpa_pool_shared_f16", GPA_POOL_PASS);
+}
+
+extern "C" int gpa_shared_set(int dtype, const void* k, const void* v, void* shared_k,
+                              void* shared_v, void* bias, float* size, int64_t B, int64_t H,
+                              int64_t S, int64_t P, int64_t pts, int64_t grid_h, int64_t grid_w,
+                              int64_t kp, int64_t D, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                              int64_t v_sb, int64_t v_sh, int64_t v_sn, void* stream) {
+  static const char* fn = "gpa_shared_set";
+  if (dtype == GPA_DTYPE_BF16)
+    return pool_run<false>(fn, k, v, shared_k, shared_v, size, nullptr, B, H, S, P, pts, grid_h,
+                           grid_w, kp, D, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, stream, bias, true);
+  if (dtype == GPA_DTYPE_F16)
+    return pool_run<true>(fn, k, v, shared_k, shared_v, size, nullptr, B, H, S, P, pts, grid_h,
+                          grid_w, kp, D, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, stream, bias, true);
+  gpa_clear_error();
+  gpa_set_error("%s: unknown dtype %d", fn, dtype);
+  return GPA_E_INVALID;
 }

@@ -52,7 +52,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from merging import _native
-from merging.fused_attention import attention_keybias, combine_by_lse
+from merging.fused_attention import attention_join, attention_keybias, attention_rows
 from merging.merge import token_merge_bipartite2d
 
 RESNET_MEAN = (0.485, 0.456, 0.406)
@@ -193,10 +193,10 @@ class Mlp(nn.Module):
 
 
 def _frame_attention(q, k, v, scale: float, backend: str) -> torch.Tensor:
-    """Plain attention, [b, H, T, D] -> [b, H, T, D] bf16."""
+    """Plain attention, [b, H, T, D] -> [b, T, H * D] bf16."""
     if backend == "sdpa":
-        return F.scaled_dot_product_attention(q, k, v)
-    return attention_keybias(q, k, v, None, scale)
+        return F.scaled_dot_product_attention(q, k, v).transpose(1, 2).flatten(2)
+    return attention_rows(q, k, v, None, scale)
 
 
 class GpaAttention(nn.Module):
@@ -285,15 +285,15 @@ class GpaAttention(nn.Module):
                 size = m(torch.ones(B, N, 1, device=x.device, dtype=torch.float32), "sum")
             bias = size.reshape(B, 1, 1, -1).log().to(q.dtype).expand(B, H, 1, k.shape[2])
             self._mark("merge")
-            out = attention_keybias(q, k, v, bias, self.scale)
+            out = attention_rows(q, k, v, bias, self.scale)
             self._mark("merged_attn")
         elif N > self.cfg.tokens_per_frame:
-            out = attention_keybias(q, k, v, None, self.scale)
+            out = attention_rows(q, k, v, None, self.scale)
             self._mark("global_attn")
         else:
             out = _frame_attention(q, k, v, self.scale, self.cfg.frame_attn)
             self._mark("frame_attn")
-        return self.proj(out.transpose(1, 2).reshape(B, N, C))
+        return self.proj(out)
 
     def _frame_special(self, q, k, v, B, N, C) -> torch.Tensor:
         """Frame attention + shared K/V set, split path (attention.py:148-176)."""
@@ -315,17 +315,16 @@ class GpaAttention(nn.Module):
             # (attention.py:178-182).
             k_f = k5.permute(0, 2, 1, 3, 4).reshape(B * S, H, P, D)
             v_f = v5.permute(0, 2, 1, 3, 4).reshape(B * S, H, P, D)
-            out = attention_keybias(q_f, k_f, v_f, None, self.scale)
-            return out.reshape(B, S, H, P, D).permute(0, 1, 3, 2, 4).reshape(B, N, C)
+            return attention_rows(q_f, k_f, v_f, None, self.scale).reshape(B, N, C)
         own_k = k5[:, :, :, pts:].permute(0, 2, 1, 3, 4).reshape(B * S, H, P - pts, D)
         own_v = v5[:, :, :, pts:].permute(0, 2, 1, 3, 4).reshape(B * S, H, P - pts, D)
         out_a, lse_a = attention_keybias(q_f, own_k, own_v, None, self.scale, return_lse=True)
         del own_k, own_v
         self._mark("frame_special_attn")
-        if kp > 0:
+        if kp > 0 and pool_kernel_applies(k, gh, gw):
+            sh_k, sh_v, bias, pool_size = _native.shared_set(k, v, S, pts, gh, gw, kp)
+        elif kp > 0:
             pooled_k, pooled_v, pool_size, _ = pool_shared_set(k, v, S, pts, gh, gw, kp)
-            if self.merge_log is not None:
-                self.merge_log.append({"kind": "pool", "frames": S, "pool_size": pool_size})
             sh_k = torch.cat([k5[:, :, :, :pts].reshape(B, H, S * pts, D), pooled_k], dim=2)
             sh_v = torch.cat([v5[:, :, :, :pts].reshape(B, H, S * pts, D), pooled_v], dim=2)
             bias = torch.zeros(B, H, 1, sh_k.shape[2], device=q.device, dtype=torch.float32)
@@ -335,12 +334,19 @@ class GpaAttention(nn.Module):
             sh_k = k5[:, :, :, :pts].reshape(B, H, S * pts, D)
             sh_v = v5[:, :, :, :pts].reshape(B, H, S * pts, D)
             bias = None
+        if kp > 0 and self.merge_log is not None:
+            self.merge_log.append({"kind": "pool", "frames": S, "pool_size": pool_size})
         self._mark("pool")
-        out_b, lse_b = attention_keybias(q, sh_k, sh_v, bias, self.scale, return_lse=True)
-        return combine_by_lse(out_a, lse_a, out_b, lse_b, S)
+        return attention_join(q, sh_k, sh_v, bias, self.scale, out_a, lse_a, S)
 
 
 POOL_KERNEL_MAX_PATCHES = 4096   # patches per frame the gpa::pool_shared kernels hold
+
+
+def pool_kernel_applies(k: torch.Tensor, grid_h: int, grid_w: int) -> bool:
+    """Whether the pooling kernels take these keys."""
+    return (grid_h * grid_w <= POOL_KERNEL_MAX_PATCHES and k.shape[-1] == 64
+            and k.dtype in (torch.bfloat16, torch.float16))
 
 
 def pool_shared_set(k: torch.Tensor, v: torch.Tensor, frames: int, pts: int, grid_h: int,
@@ -353,8 +359,7 @@ def pool_shared_set(k: torch.Tensor, v: torch.Tensor, frames: int, pts: int, gri
     reference's own torch ops on the device (`pool_shared_torch`).
     Returns (pooled_k, pooled_v [B, H, S*npool, D], size [B, H, S, npool]
     fp32, assign [B, H, S, grid_h*grid_w] or an empty tensor)."""
-    if (grid_h * grid_w <= POOL_KERNEL_MAX_PATCHES and k.shape[-1] == 64
-            and k.dtype in (torch.bfloat16, torch.float16)):
+    if pool_kernel_applies(k, grid_h, grid_w):
         return _native.pool_shared(k, v, frames, pts, grid_h, grid_w, kp, want_assign)
     B, H, N, D = k.shape
     P = N // frames

@@ -39,7 +39,7 @@ from typing import Optional, Tuple
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libgpa_mi355x.so"
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 GPA_OK = 0
 GPA_E_INVALID = -1
@@ -114,6 +114,13 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.gpa_attn_keybias_bf16_noalloc.restype = ctypes.c_int
     lib.gpa_attn_keybias_bf16_noalloc.argtypes = (
         lib.gpa_attn_keybias_bf16.argtypes[:-4] + [ctypes.c_float, _vp])   # no workspace
+    lib.gpa_attn_keybias_join.restype = ctypes.c_int
+    lib.gpa_attn_keybias_join.argtypes = [
+        ctypes.c_int, *lib.gpa_attn_keybias_bf16.argtypes[:8],   # dtype, q .. bias strides
+        _vp, _vp, _i64, _vp,           # other_o, other_lse, P, o
+        *lib.gpa_attn_keybias_bf16.argtypes[10:27],              # B .. o strides
+        _vp, ctypes.c_size_t, ctypes.c_float, _vp,
+    ]
     lib.gpa_lse_combine_bf16.restype = ctypes.c_int
     lib.gpa_lse_combine_bf16.argtypes = [_vp] * 5 + [_i64] * 5 + [_i64] * 16 + [_i64] * 3 + [_vp]
     lib.gpa_lse_combine_f16.restype = ctypes.c_int
@@ -139,6 +146,8 @@ def _bind(lib: ctypes.CDLL) -> None:
     ]
     lib.gpa_pool_shared_f16.restype = ctypes.c_int
     lib.gpa_pool_shared_f16.argtypes = lib.gpa_pool_shared_bf16.argtypes
+    lib.gpa_shared_set.restype = ctypes.c_int
+    lib.gpa_shared_set.argtypes = [ctypes.c_int, *lib.gpa_pool_shared_bf16.argtypes]
     lib.gpa_merge_metric_bf16.restype = ctypes.c_int
     lib.gpa_merge_metric_bf16.argtypes = [
         _vp, ctypes.c_int,             # metric, metric dtype
@@ -207,7 +216,7 @@ def exported_symbols() -> Tuple[str, ...]:
             "gpa_pool_shared_bf16", "gpa_merge_metric_bf16", "gpa_sim_argmax_f16",
             "gpa_attn_keybias_f16", "gpa_residual_layernorm_bf16",
             "gpa_attn_keybias_bf16_noalloc", "gpa_lse_combine_f16", "gpa_qk_norm_rope_f16",
-            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16")
+            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16", "gpa_shared_set", "gpa_attn_keybias_join")
 
 
 def _check(rc: int, what: str) -> None:
@@ -376,9 +385,11 @@ _ATTN_BOUND_BYTES = 16
 ATTN_FLAG_LAZY, ATTN_FLAG_TILE0, ATTN_FLAG_RERUN = 1, 2, 4
 
 
-def _attn_run(q, k, v, bias, sm_scale, return_lse):
+def _attn_run(q, k, v, bias, sm_scale, return_lse, rows=False, join=None):
     """Validate, allocate and launch gpa_attn_keybias_{bf16,f16}; returns
-    (o, lse, workspace) with the workspace as the kernel left it."""
+    (o, lse, workspace) with the workspace as the kernel left it.  With `rows`
+    o is a [B, H, M, D] view of a contiguous [B, M, H, D]; join (o, lse, P):
+    gpa_attn_keybias_join with that other attention."""
     tensors = [q, k, v] + ([bias] if bias is not None else [])
     dev = _require_gpu(*tensors)
     if q.dtype not in (torch.bfloat16, torch.float16):
@@ -412,7 +423,8 @@ def _attn_run(q, k, v, bias, sm_scale, return_lse):
                      torch.float16: GPA_BIAS_F16}[bx.dtype]
         bias_ptr = bx.data_ptr()
         bsb, bsh, bsn = _st(bx, 0), _st(bx, 1), _st(bx, 3)
-    o = torch.empty(B, H, M, D, device=dev, dtype=q.dtype)
+    o = (torch.empty(B, M, H, D, device=dev, dtype=q.dtype).transpose(1, 2) if rows
+         else torch.empty(B, H, M, D, device=dev, dtype=q.dtype))
     lse = (torch.empty(B, H, M, device=dev, dtype=torch.float32) if return_lse
            else torch.empty(0, device=dev, dtype=torch.float32))
     if B == 0 or H == 0 or M == 0:
@@ -421,17 +433,20 @@ def _attn_run(q, k, v, bias, sm_scale, return_lse):
     ws_bytes = L.gpa_attn_keybias_workspace_bytes(B, H, M, N)
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
     with _on(dev):
-        fn = L.gpa_attn_keybias_f16 if q.dtype == torch.float16 else L.gpa_attn_keybias_bf16
-        rc = fn(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), bias_ptr, bias_kind, bsb, bsh, bsn,
-            o.data_ptr(), lse.data_ptr() if return_lse else None,
-            B, H, M, N, D,
-            _st(q, 0), _st(q, 1), _rs(q, 2),
-            _st(k, 0), _st(k, 1), _rs(k, 2),
-            _st(v, 0), _st(v, 1), _rs(v, 2),
-            _st(o, 0), _st(o, 1), _rs(o, 2),
-            _st(lse, 0) if return_lse else 0, _st(lse, 1) if return_lse else 0,
-            ws.data_ptr(), ws_bytes, float(sm_scale), _stream(dev))
+        operands = (q.data_ptr(), k.data_ptr(), v.data_ptr(), bias_ptr, bias_kind, bsb, bsh, bsn)
+        shape = (B, H, M, N, D,
+                 _st(q, 0), _st(q, 1), _rs(q, 2),
+                 _st(k, 0), _st(k, 1), _rs(k, 2),
+                 _st(v, 0), _st(v, 1), _rs(v, 2),
+                 _st(o, 0), _st(o, 1), _rs(o, 2))
+        tail = (ws.data_ptr(), ws_bytes, float(sm_scale), _stream(dev))
+        if join is not None:
+            rc = L.gpa_attn_keybias_join(_DTYPE_CODES[q.dtype], *operands, join[0].data_ptr(),
+                                         join[1].data_ptr(), join[2], o.data_ptr(), *shape, *tail)
+        else:
+            fn = L.gpa_attn_keybias_f16 if q.dtype == torch.float16 else L.gpa_attn_keybias_bf16
+            rc = fn(*operands, o.data_ptr(), lse.data_ptr() if return_lse else None, *shape,
+                    _st(lse, 0) if return_lse else 0, _st(lse, 1) if return_lse else 0, *tail)
     _check(rc, "gpa::attn_keybias")
     return o, lse, ws
 
@@ -482,6 +497,55 @@ def _attn_keybias_fake(q, k, v, bias, sm_scale, return_lse):
     o = q.new_empty(B, H, M, D)
     lse = q.new_empty((B, H, M) if return_lse else (0,), dtype=torch.float32)
     return o, lse
+
+
+@_op
+def attn_keybias_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                      bias: Optional[torch.Tensor], sm_scale: float) -> torch.Tensor:
+    """The attention's output [B, H, M, D] as the [B, M, H*D] rows of an output
+    projection, written so by the kernel (transposed afterwards it was another
+    pass: 11 us of a 6-frame block)."""
+    B, H, M, D = q.shape
+    o, _, _ = _attn_run(q, k, v, bias, sm_scale, False, rows=True)
+    return o.transpose(1, 2).reshape(B, M, H * D)
+
+
+@_fake("attn_keybias_rows")
+def _attn_keybias_rows_fake(q, k, v, bias, sm_scale):
+    B, H, M, D = q.shape
+    return q.new_empty(B, M, H * D)
+
+
+@_op
+def attn_keybias_join(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                      bias: Optional[torch.Tensor], sm_scale: float, other_o: torch.Tensor,
+                      other_lse: torch.Tensor, frames: int) -> torch.Tensor:
+    """The attention of q [B, H, S*P, 64] over k and v joined by LSE with another
+    one of the same queries over further keys, as the own-frame call returns it:
+    other_o [B*S, H, P, 64] in q's dtype, other_lse [B*S, H, P] fp32 (log2).
+    Returns [B, S*P, H*64] (gpa::lse_combine of the two, whose second half
+    stays in fp32)."""
+    _require_gpu(q, other_o, other_lse)
+    B, H, M, D = q.shape
+    S = int(frames)
+    P = M // S if S > 0 else 0
+    if S <= 0 or P * S != M or D != 64 or other_o.dtype != q.dtype \
+            or other_lse.dtype != torch.float32 or other_o.shape != (B * S, H, P, D) \
+            or other_lse.shape != (B * S, H, P):
+        raise ValueError(f"gpa::attn_keybias_join: q {q.dtype} {tuple(q.shape)}, other_o "
+                         f"{other_o.dtype} {tuple(other_o.shape)}, other_lse {other_lse.dtype} "
+                         f"{tuple(other_lse.shape)}, frames {frames}")
+    other_o, other_lse = other_o.contiguous(), other_lse.contiguous()
+    if other_o.data_ptr() % 16:
+        other_o = other_o.clone()
+    o, _, _ = _attn_run(q, k, v, bias, sm_scale, False, rows=True, join=(other_o, other_lse, P))
+    return o.transpose(1, 2).reshape(B, M, H * D)
+
+
+@_fake("attn_keybias_join")
+def _attn_keybias_join_fake(q, k, v, bias, sm_scale, other_o, other_lse, frames):
+    B, H, M, D = q.shape
+    return q.new_empty(B, M, H * D)
 
 
 _MERGE_DTYPES = _DTYPE_CODES
@@ -788,6 +852,53 @@ def _pool_shared_fake(k, v, frames, pts, grid_h, grid_w, kp, want_assign):
             k.new_empty(B, H, frames, npool, dtype=torch.float32),
             k.new_empty((B, H, frames, grid_h * grid_w) if want_assign else (0,),
                         dtype=torch.int32))
+
+
+@_op
+def shared_set(k: torch.Tensor, v: torch.Tensor, frames: int, pts: int, grid_h: int, grid_w: int,
+               kp: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """The shared set of a frame-special block from k, v [B, H, S*P, 64] (both
+    bf16 or both fp16): keys and values [B, H, n, 64] (every frame's `pts`
+    special tokens, then every frame's pooled summaries), the bias
+    [B, H, 1, n] in their format (0, then log(size)) and the pool sizes
+    [B, H, S, npool] fp32."""
+    dev = _require_gpu(k, v)
+    if k.dtype not in (torch.bfloat16, torch.float16) or v.dtype != k.dtype or k.dim() != 4 \
+            or k.shape != v.shape:
+        raise ValueError(f"gpa::shared_set: k and v must both be bf16 or fp16 [B,H,N,64], got "
+                         f"{k.dtype} {tuple(k.shape)} and {v.dtype} {tuple(v.shape)}")
+    B, H, N, D = k.shape
+    S = int(frames)
+    if kp <= 0 or grid_h <= 0 or grid_w <= 0 or S <= 0 or N % S != 0:
+        raise ValueError(f"gpa::shared_set: {N} tokens in {S} frames, grid {grid_h}x{grid_w}, kp {kp}")
+    npool = -(-int(grid_h) // int(kp)) * -(-int(grid_w) // int(kp))
+    n = S * (pts + npool)
+    if not _rows_ok(k, 8):
+        k = k.contiguous()
+    if not _rows_ok(v, 8):
+        v = v.contiguous()
+    sk = torch.empty(B, H, n, D, device=dev, dtype=k.dtype)
+    sv = torch.empty(B, H, n, D, device=dev, dtype=k.dtype)
+    bias = torch.empty(B, H, 1, n, device=dev, dtype=k.dtype)
+    size = torch.empty(B, H, S, npool, device=dev, dtype=torch.float32)
+    if sk.numel() == 0:
+        return sk, sv, bias, size
+    with _on(dev):
+        rc = lib().gpa_shared_set(
+            _DTYPE_CODES[k.dtype], k.data_ptr(), v.data_ptr(), sk.data_ptr(), sv.data_ptr(),
+            bias.data_ptr(), size.data_ptr(), B, H, S, N // S, pts, grid_h, grid_w, kp, D,
+            _st(k, 0), _st(k, 1), _rs(k, 2), _st(v, 0), _st(v, 1), _rs(v, 2), _stream(dev))
+    _check(rc, "gpa::shared_set")
+    return sk, sv, bias, size
+
+
+@_fake("shared_set")
+def _shared_set_fake(k, v, frames, pts, grid_h, grid_w, kp):
+    B, H, N, D = k.shape
+    npool = -(-grid_h // kp) * -(-grid_w // kp)
+    n = frames * (pts + npool)
+    return (k.new_empty(B, H, n, D), k.new_empty(B, H, n, D), k.new_empty(B, H, 1, n),
+            k.new_empty(B, H, frames, npool, dtype=torch.float32))
 
 
 # --------------------------------------------------------------------------

@@ -15,11 +15,13 @@ frame-special split path of vggt/layers/attention.py:148-176.
 """
 from __future__ import annotations
 
+from typing import Optional
+
 import torch
 
 from . import _native
 
-__all__ = ["attention_keybias", "combine_by_lse", "LOG2E"]
+__all__ = ["attention_keybias", "attention_join", "attention_rows", "combine_by_lse", "LOG2E"]
 
 LOG2E = 1.4426950408889634
 
@@ -28,6 +30,19 @@ def _autocast_dtype() -> torch.dtype:
     if torch.is_autocast_enabled("cuda"):
         return torch.get_autocast_dtype("cuda")
     return torch.bfloat16
+
+
+def _operands(q, k, v, bias):
+    if q.dtype == torch.float32:
+        dt = _autocast_dtype()
+        q, k, v = q.to(dt), k.to(dt), v.to(dt)
+        bias = None if bias is None else bias.to(dt)
+    if q.dtype not in (torch.bfloat16, torch.float16):
+        raise NotImplementedError(
+            f"attention_keybias: {q.dtype} is not supported; the gfx950 kernels run bf16 and fp16")
+    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+        raise ValueError("attention_keybias expects [B, H, T, D] q/k/v")
+    return q, k.to(q.dtype), v.to(q.dtype), bias
 
 
 def attention_keybias(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -40,19 +55,28 @@ def attention_keybias(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     [B, H, M] fp32 log2 softmax denominators.  `bias` may be None (plain
     attention).
     """
-    if q.dtype == torch.float32:
-        dt = _autocast_dtype()
-        q, k, v = q.to(dt), k.to(dt), v.to(dt)
-        bias = None if bias is None else bias.to(dt)
-    if q.dtype not in (torch.bfloat16, torch.float16):
-        raise NotImplementedError(
-            f"attention_keybias: {q.dtype} is not supported; the gfx950 kernels run bf16 and fp16")
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise ValueError("attention_keybias expects [B, H, T, D] q/k/v")
-    v = v.to(q.dtype)
-    k = k.to(q.dtype)
+    q, k, v, bias = _operands(q, k, v, bias)
     o, lse = _native.attn_keybias(q, k, v, bias, float(sm_scale), bool(return_lse))
     return (o, lse) if return_lse else o
+
+
+def attention_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                   bias: Optional[torch.Tensor], sm_scale: float) -> torch.Tensor:
+    """`attention_keybias` as the [B, M, H*D] rows the output projection takes."""
+    return _native.attn_keybias_rows(*_operands(q, k, v, bias), float(sm_scale))
+
+
+def attention_join(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                   bias: Optional[torch.Tensor], sm_scale: float, out_a: torch.Tensor,
+                   lse_a: torch.Tensor, frames: int) -> torch.Tensor:
+    """`attention_keybias` of all queries over the shared keys and
+    `combine_by_lse` with the own-frame half (out_a, lse_a), in one pass at head
+    dim 64, where the shared half then stays in fp32."""
+    q, k, v, bias = _operands(q, k, v, bias)
+    if q.shape[-1] == 64 and out_a.dtype == q.dtype:
+        return _native.attn_keybias_join(q, k, v, bias, float(sm_scale), out_a, lse_a, int(frames))
+    out_b, lse_b = _native.attn_keybias(q, k, v, bias, float(sm_scale), True)
+    return combine_by_lse(out_a, lse_a, out_b, lse_b, frames)
 
 
 def combine_by_lse(out_a: torch.Tensor, lse_a: torch.Tensor, out_b: torch.Tensor,

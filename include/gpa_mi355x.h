@@ -58,7 +58,7 @@
 extern "C" {
 #endif
 
-#define GPA_ABI_VERSION 16
+#define GPA_ABI_VERSION 17
 
 enum {
   GPA_OK = 0,
@@ -183,6 +183,28 @@ int gpa_attn_keybias_f16(const void* q, const void* k, const void* v,
                          int64_t lse_sb, int64_t lse_sh,
                          void* workspace, size_t workspace_bytes,
                          float sm_scale, void* stream);
+
+/* The second attention of a split key set, joined by LSE with the first:
+ *   a = the attention over k, v and bias as above, with LSE la
+ *   o = (other_o 2^(other_lse - m) + a 2^(la - m)) / (2^(other_lse - m) + 2^(la - m)),
+ *   m = max(other_lse, la)
+ * in fp32, rounded once.  dtype GPA_DTYPE_BF16 or GPA_DTYPE_F16 (q, k, v, o
+ * and other_o), D = 64.  other_o [B*M/P, H, P, 64] and other_lse
+ * [B*M/P, H, P] (log2, fp32) are contiguous: query n of batch b is row n % P
+ * of frame b*M/P + n / P; M a multiple of P.  Replaces the second call and
+ * the combination of vggt/layers/attention.py:157-176. */
+int gpa_attn_keybias_join(int dtype, const void* q, const void* k, const void* v,
+                          const void* bias, int bias_kind,
+                          int64_t bias_sb, int64_t bias_sh, int64_t bias_sn,
+                          const void* other_o, const float* other_lse, int64_t P,
+                          void* o,
+                          int64_t B, int64_t H, int64_t M, int64_t N, int64_t D,
+                          int64_t q_sb, int64_t q_sh, int64_t q_sm,
+                          int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                          int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                          int64_t o_sb, int64_t o_sh, int64_t o_sm,
+                          void* workspace, size_t workspace_bytes,
+                          float sm_scale, void* stream);
 
 /* Bytes of the device-resident scratch array behind
  * gpa_attn_keybias_bf16_noalloc (one per GPU, held until the process ends). */
@@ -381,6 +403,22 @@ int gpa_pool_shared_f16(const void* k, const void* v, void* pooled_k, void* pool
                         int64_t P, int64_t pts, int64_t grid_h, int64_t grid_w, int64_t kp,
                         int64_t D, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                         int64_t v_sb, int64_t v_sh, int64_t v_sn, void* stream);
+
+/*
+ * The whole shared set of a frame-special block from k and v (dtype
+ * GPA_DTYPE_BF16 or GPA_DTYPE_F16), n = S*(pts + npool) keys per (b, h): rows
+ * s*pts + i are the special tokens (k[b, h, s*P + i, :], bias 0), row
+ * S*pts + s*npool + g the pooled summary above (bias log(size), rounded to
+ * dtype; -inf for an empty group).  shared_k / shared_v: contiguous
+ * [B, H, n, 64], bias [B, H, n], all of dtype; size as above.  Same limits.
+ * Replaces vggt/layers/attention.py:113-146 (`_pool`, the concatenations and
+ * the bias).
+ */
+int gpa_shared_set(int dtype, const void* k, const void* v, void* shared_k, void* shared_v,
+                   void* bias, float* size, int64_t B, int64_t H, int64_t S, int64_t P,
+                   int64_t pts, int64_t grid_h, int64_t grid_w, int64_t kp, int64_t D,
+                   int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t v_sb, int64_t v_sh,
+                   int64_t v_sn, void* stream);
 
 /*
  * Front end of the bipartite merge: for every batch b and output row j,
