@@ -51,8 +51,9 @@ constexpr int kHeadDim = 64;
 struct QkArgs {
   const uint16_t* qkv;
   int64_t sb, sn, k_offset;
-  const float* w;      // [2][64]: q then k
-  const float* beta;   // [2][64]
+  const void* w[2];     // q's and k's LayerNorm weights [64]
+  const void* beta[2];  // and biases
+  int param;            // their GPA_DTYPE_* format
   float eps;
   const int32_t* pos;  // [period][2] or null (no rotation)
   int64_t period;
@@ -84,6 +85,21 @@ __device__ __forceinline__ float group_sum8(float v) {
   return v;
 }
 
+// Eight LayerNorm parameters in fp32.  They are read in the model's own
+// format: gathered into one fp32 array beforehand they were four launches per
+// block (~12 us beside the 22 us of this kernel at 6 frames).
+__device__ __forceinline__ void load_params(const void* p, int kind, int at, float (&x)[8]) {
+  if (kind == GPA_DTYPE_F32) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = static_cast<const float*>(p)[at + i];
+  } else {
+    const bf16x8 v = *reinterpret_cast<const bf16x8*>(static_cast<const uint16_t*>(p) + at);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      x[i] = kind == GPA_DTYPE_BF16 ? half_to_f32<false>(v[i]) : half_to_f32<true>(v[i]);
+  }
+}
+
 // F16: the projection and the 16-bit outputs are fp16 (the fp16-autocast
 // stack) instead of bf16; the arithmetic is the same fp32.
 template <bool F16>
@@ -113,8 +129,9 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(QkArgs a) {
         reinterpret_cast<const u32x4*>(a.qkv + (int64_t)b * a.sb + (int64_t)n * a.sn + col);
     xv[r] = __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(src));
   }
-  const float* w = a.w + which * kHeadDim + c * 8;
-  const float* be = a.beta + which * kHeadDim + c * 8;
+  float w[8], be[8];
+  load_params(a.w[which], a.param, c * 8, w);
+  load_params(a.beta[which], a.param, c * 8, be);
   void* out = which ? a.k_out : a.q_out;
   const bool out_f32 = which ? a.k_f32 : a.q_f32;
 
@@ -184,8 +201,9 @@ namespace {
 // messages.
 template <bool F16>
 int qk_run(const char* fn, const void* qkv, int64_t B, int64_t N, int64_t H, int64_t D,
-           int64_t qkv_sb, int64_t qkv_sn, int64_t k_offset, const float* ln_weight,
-           const float* ln_bias, float eps, const int32_t* pos, int64_t period,
+           int64_t qkv_sb, int64_t qkv_sn, int64_t k_offset, const void* q_weight,
+           const void* k_weight, const void* q_bias, const void* k_bias, int param_dtype,
+           float eps, const int32_t* pos, int64_t period,
            const float* rope_cs, int64_t npos, void* q_out, int q_dtype, void* k_out,
            int k_dtype, void* stream) {
   gpa_clear_error();
@@ -198,7 +216,7 @@ int qk_run(const char* fn, const void* qkv, int64_t B, int64_t N, int64_t H, int
     return GPA_E_UNSUPPORTED;
   }
   if (B == 0 || N == 0 || H == 0) return GPA_OK;
-  if (!qkv || !ln_weight || !ln_bias || !q_out || !k_out) {
+  if (!qkv || !q_weight || !k_weight || !q_bias || !k_bias || !q_out || !k_out) {
     gpa_set_error("%s: null pointer", fn);
     return GPA_E_INVALID;
   }
@@ -212,6 +230,15 @@ int qk_run(const char* fn, const void* qkv, int64_t B, int64_t N, int64_t H, int
       gpa_set_error("%s: output dtype %d is not fp32 or %s", fn, dt, F16 ? "fp16" : "bf16");
       return GPA_E_UNSUPPORTED;
     }
+  }
+  if (param_dtype != GPA_DTYPE_F32 && param_dtype != GPA_DTYPE_BF16 && param_dtype != GPA_DTYPE_F16) {
+    gpa_set_error("%s: unknown parameter dtype %d", fn, param_dtype);
+    return GPA_E_INVALID;
+  }
+  if (param_dtype != GPA_DTYPE_F32 &&
+      (((uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)q_bias | (uintptr_t)k_bias) % 16)) {
+    gpa_set_error("%s: 16-bit LayerNorm parameters must be 16-byte aligned", fn);
+    return GPA_E_INVALID;
   }
   const bool aligned = (uintptr_t)qkv % 16 == 0 && (uintptr_t)q_out % 16 == 0 &&
                        (uintptr_t)k_out % 16 == 0 && (B == 1 || qkv_sb % 8 == 0) &&
@@ -228,7 +255,8 @@ int qk_run(const char* fn, const void* qkv, int64_t B, int64_t N, int64_t H, int
   QkArgs a{};
   a.qkv = (const uint16_t*)qkv;
   a.sb = qkv_sb; a.sn = qkv_sn; a.k_offset = k_offset;
-  a.w = ln_weight; a.beta = ln_bias; a.eps = eps;
+  a.w[0] = q_weight; a.w[1] = k_weight; a.beta[0] = q_bias; a.beta[1] = k_bias;
+  a.param = param_dtype; a.eps = eps;
   a.pos = pos; a.period = period; a.cs = rope_cs; a.npos = (int32_t)npos;
   a.q_out = q_out; a.k_out = k_out;
   a.q_f32 = q_dtype == GPA_DTYPE_F32; a.k_f32 = k_dtype == GPA_DTYPE_F32;
@@ -257,7 +285,8 @@ int qk_run(const char* fn, const void* qkv, int64_t B, int64_t N, int64_t H, int
       const int32_t *pos, int64_t period, const float *rope_cs, int64_t npos, void *q_out,    \
       int q_dtype, void *k_out, int k_dtype, void *stream
 #define GPA_QK_PASS                                                                          \
-  qkv, B, N, H, D, qkv_sb, qkv_sn, k_offset, ln_weight, ln_bias, eps, pos, period, rope_cs,  \
+  qkv, B, N, H, D, qkv_sb, qkv_sn, k_offset, ln_weight, ln_weight ? ln_weight + 64 : nullptr, \
+      ln_bias, ln_bias ? ln_bias + 64 : nullptr, GPA_DTYPE_F32, eps, pos, period, rope_cs,     \
       npos, q_out, q_dtype, k_out, k_dtype, stream
 
 extern "C" int gpa_qk_norm_rope_bf16(GPA_QK_ARGS) {
@@ -266,4 +295,26 @@ extern "C" int gpa_qk_norm_rope_bf16(GPA_QK_ARGS) {
 
 extern "C" int gpa_qk_norm_rope_f16(GPA_QK_ARGS) {
   return qk_run<true>("gpa_qk_norm_rope_f16", GPA_QK_PASS);
+}
+
+extern "C" int gpa_qk_norm_rope_params(int dtype, const void* qkv, int64_t B, int64_t N, int64_t H,
+                                       int64_t D, int64_t qkv_sb, int64_t qkv_sn,
+                                       int64_t k_offset, const void* q_weight,
+                                       const void* k_weight, const void* q_bias,
+                                       const void* k_bias, int param_dtype, float eps,
+                                       const int32_t* pos, int64_t period, const float* rope_cs,
+                                       int64_t npos, void* q_out, int q_dtype, void* k_out,
+                                       int k_dtype, void* stream) {
+  static const char* fn = "gpa_qk_norm_rope_params";
+  if (dtype == GPA_DTYPE_BF16)
+    return qk_run<false>(fn, qkv, B, N, H, D, qkv_sb, qkv_sn, k_offset, q_weight, k_weight, q_bias,
+                         k_bias, param_dtype, eps, pos, period, rope_cs, npos, q_out, q_dtype,
+                         k_out, k_dtype, stream);
+  if (dtype == GPA_DTYPE_F16)
+    return qk_run<true>(fn, qkv, B, N, H, D, qkv_sb, qkv_sn, k_offset, q_weight, k_weight, q_bias,
+                        k_bias, param_dtype, eps, pos, period, rope_cs, npos, q_out, q_dtype,
+                        k_out, k_dtype, stream);
+  gpa_clear_error();
+  gpa_set_error("%s: unknown dtype %d", fn, dtype);
+  return GPA_E_INVALID;
 }

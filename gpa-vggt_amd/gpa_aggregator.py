@@ -240,10 +240,9 @@ class GpaAttention(nn.Module):
             if qkv.dtype not in (torch.bfloat16, torch.float16):
                 raise ValueError("the fused qk-norm/RoPE kernel takes a bf16 or fp16 "
                                  "projection (run the model under bf16 or fp16 autocast)")
-            ln_w = torch.stack((self.q_norm.weight, self.k_norm.weight))
-            ln_b = torch.stack((self.q_norm.bias, self.k_norm.bias))
-            q, k = _native.qk_norm_rope(
-                qkv, ln_w, ln_b, self.q_norm.eps, None if rope is None else rope.pos,
+            q, k = _native.qk_norm_rope_params(
+                qkv, self.q_norm.weight, self.k_norm.weight, self.q_norm.bias, self.k_norm.bias,
+                self.q_norm.eps, None if rope is None else rope.pos,
                 None if rope is None else rope.cs, H, False, k_f32)
             return q, k, v
         if rope is not None:
@@ -428,19 +427,49 @@ class Block(nn.Module):
         return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == dt
 
     def forward(self, x, rope: Optional[RopeTable] = None, global_merging=None):
+        return self.step(x, None, rope, global_merging)[0]
+
+    def step(self, x, ln1: Optional[torch.Tensor], rope: Optional[RopeTable] = None,
+             global_merging=None, following: Optional["Block"] = None):
+        """The block as one of a chain: ln1, if given, is this block's first
+        LayerNorm of x; returns the output and, where `following` takes it
+        fused, that block's first LayerNorm of it (else None)."""
         if self._fused_ok(x):
             # block.py:84-96 with the elementwise steps fused: LayerNorm 1 to
-            # the 16-bit format; x + ls1(attn) with LayerNorm 2 in one pass;
-            # x + ls2(mlp).
+            # the 16-bit format (of the first block of a chain); x + ls1(attn)
+            # with LayerNorm 2 in one pass; x + ls2(mlp) with the next block's
+            # LayerNorm 1, which saves that its read of the stream and a launch.
             rl = _native.residual_layernorm
-            _, ln1 = rl(x, None, None, self.norm1.weight, self.norm1.bias, self.norm1.eps, False)
-            a = self.attn(ln1, rope, global_merging)
+            if ln1 is None:
+                _, ln1 = rl(x, None, None, self.norm1.weight, self.norm1.bias, self.norm1.eps,
+                            False)
+            a = self.attn(ln1.view(x.shape), rope, global_merging)
             h, ln2 = rl(x, a, self.ls1.gamma, self.norm2.weight, self.norm2.bias,
                         self.norm2.eps, True)
-            out, _ = rl(h, self.mlp(ln2), self.ls2.gamma, None, None, 0.0, True)
-            return out
+            nxt = following.norm1 if following is not None and following._fused_ok(x) else None
+            if nxt is None:
+                return rl(h, self.mlp(ln2), self.ls2.gamma, None, None, 0.0, True)[0], None
+            return rl(h, self.mlp(ln2), self.ls2.gamma, nxt.weight, nxt.bias, nxt.eps, True)
         x = x + self.ls1(self.attn(self.norm1(x), rope, global_merging))
-        return x + self.ls2(self.mlp(self.norm2(x)))
+        return x + self.ls2(self.mlp(self.norm2(x))), None
+
+
+def _chainable(blk: nn.Module) -> bool:
+    """A plain Block whose call does no more than its `step`: no hooks, no
+    replaced forward."""
+    mod = torch.nn.modules.module
+    return (type(blk) is Block and "forward" not in blk.__dict__ and not blk._forward_hooks
+            and not blk._forward_pre_hooks and not mod._global_forward_hooks
+            and not mod._global_forward_pre_hooks)
+
+
+def _chain_step(blk, x, ln1, rope=None, global_merging=None, following=None):
+    """One block of a chain: `Block.step`, or the module call where something
+    hangs on it (and then without the LayerNorms shared between blocks)."""
+    if not _chainable(blk):
+        return blk(x, rope, global_merging), None
+    return blk.step(x, ln1, rope, global_merging,
+                    following if following is not None and _chainable(following) else None)
 
 
 class DinoV2Reg(nn.Module):
@@ -480,8 +509,9 @@ class DinoV2Reg(nn.Module):
         x = x + self.pos_embed.to(x.dtype)
         x = torch.cat((x[:, :1], self.register_tokens.expand(x.shape[0], -1, -1).to(x.dtype),
                        x[:, 1:]), dim=1)
-        for blk in self.blocks:
-            x = blk(x)
+        ln = None
+        for blk, following in zip(self.blocks, [*self.blocks[1:], None]):
+            x, ln = _chain_step(blk, x, ln, following=following)
         return self.norm(x)[:, 1 + self.nreg:]
 
 
@@ -568,12 +598,16 @@ class GpaAggregator(nn.Module):
         P, C = tokens.shape[1], tokens.shape[2]
         rope = self.rope_table(images.device)
         outputs = []
+        ln = None
         for i in range(self.cfg.depth):
-            tokens = self.frame_blocks[i](tokens.view(B * S, P, C), rope)
+            tokens, ln = _chain_step(self.frame_blocks[i], tokens.view(B * S, P, C), ln, rope,
+                                     following=self.global_blocks[i])
             self._mark("frame_block")
             frame_out = tokens.view(B, S, P, C)
-            tokens = self.global_blocks[i](tokens.view(B, S * P, C), rope,
-                                           self.cfg.global_merging(i))
+            tokens, ln = _chain_step(
+                self.global_blocks[i], tokens.view(B, S * P, C), ln, rope,
+                self.cfg.global_merging(i),
+                following=self.frame_blocks[i + 1] if i + 1 < self.cfg.depth else None)
             self._mark(f"global_block_{self.cfg.block_kind(i)}")
             if i in self.cfg.dpt_blocks:
                 outputs.append(torch.cat((frame_out, tokens.view(B, S, P, C)), dim=-1))

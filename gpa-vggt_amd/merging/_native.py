@@ -39,7 +39,7 @@ from typing import Optional, Tuple
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libgpa_mi355x.so"
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 GPA_OK = 0
 GPA_E_INVALID = -1
@@ -136,6 +136,12 @@ def _bind(lib: ctypes.CDLL) -> None:
     ]
     lib.gpa_qk_norm_rope_f16.restype = ctypes.c_int
     lib.gpa_qk_norm_rope_f16.argtypes = lib.gpa_qk_norm_rope_bf16.argtypes
+    lib.gpa_qk_norm_rope_params.restype = ctypes.c_int
+    lib.gpa_qk_norm_rope_params.argtypes = [
+        ctypes.c_int, *lib.gpa_qk_norm_rope_bf16.argtypes[:8],   # dtype, qkv .. k_offset
+        _vp, _vp, _vp, _vp, ctypes.c_int,                        # parameters and their dtype
+        *lib.gpa_qk_norm_rope_bf16.argtypes[10:],                # eps ..
+    ]
     lib.gpa_pool_shared_bf16.restype = ctypes.c_int
     lib.gpa_pool_shared_bf16.argtypes = [
         _vp, _vp, _vp, _vp, _vp, _vp,  # k, v, pooled_k, pooled_v, size, assign
@@ -216,7 +222,8 @@ def exported_symbols() -> Tuple[str, ...]:
             "gpa_pool_shared_bf16", "gpa_merge_metric_bf16", "gpa_sim_argmax_f16",
             "gpa_attn_keybias_f16", "gpa_residual_layernorm_bf16",
             "gpa_attn_keybias_bf16_noalloc", "gpa_lse_combine_f16", "gpa_qk_norm_rope_f16",
-            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16", "gpa_shared_set", "gpa_attn_keybias_join")
+            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16", "gpa_shared_set", "gpa_attn_keybias_join",
+            "gpa_qk_norm_rope_params")
 
 
 def _check(rc: int, what: str) -> None:
@@ -747,6 +754,35 @@ def qk_norm_rope(qkv: torch.Tensor, ln_w: torch.Tensor, ln_b: torch.Tensor, eps:
     [npos, 16, 2] fp32 (cos, sin) tables, or both None for no rotation.
     """
     dev = _require_gpu(qkv, ln_w, ln_b)
+    w = ln_w.to(device=dev, dtype=torch.float32).contiguous()
+    bb = ln_b.to(device=dev, dtype=torch.float32).contiguous()
+    if w.numel() != 128 or bb.numel() != 128:
+        raise ValueError("gpa::qk_norm_rope: ln_w and ln_b hold the q and k weights, 2 x 64")
+    w, bb = w.view(2, 64), bb.view(2, 64)
+    return _qk_run(qkv, (w[0], w[1], bb[0], bb[1]), eps, pos, rope_cs, heads, q_f32, k_f32)
+
+
+@_op
+def qk_norm_rope_params(qkv: torch.Tensor, q_w: torch.Tensor, k_w: torch.Tensor,
+                        q_b: torch.Tensor, k_b: torch.Tensor, eps: float,
+                        pos: Optional[torch.Tensor], rope_cs: Optional[torch.Tensor], heads: int,
+                        q_f32: bool, k_f32: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    """gpa::qk_norm_rope with the four LayerNorm parameters [64] as the model
+    holds them."""
+    params = (q_w, k_w, q_b, k_b)
+    dev = _require_gpu(qkv, *params)
+    if any(p.numel() != 64 for p in params):
+        raise ValueError("gpa::qk_norm_rope: a LayerNorm parameter holds 64 values, got "
+                         f"{[tuple(p.shape) for p in params]}")
+    if any(p.dtype != q_w.dtype or p.dtype not in _DTYPE_CODES or not p.is_contiguous()
+           or p.data_ptr() % 16 for p in params):
+        params = tuple(p.to(device=dev, dtype=torch.float32).contiguous() for p in params)
+    return _qk_run(qkv, params, eps, pos, rope_cs, heads, q_f32, k_f32)
+
+
+def _qk_run(qkv, params, eps, pos, rope_cs, heads, q_f32, k_f32):
+    """Validate, allocate and launch gpa_qk_norm_rope_params."""
+    dev = qkv.device
     if qkv.dtype not in (torch.bfloat16, torch.float16) or qkv.dim() != 3:
         raise ValueError(f"gpa::qk_norm_rope: qkv must be bf16 or fp16 [B, N, 3C], got "
                          f"{qkv.dtype} {tuple(qkv.shape)}")
@@ -754,10 +790,6 @@ def qk_norm_rope(qkv: torch.Tensor, ln_w: torch.Tensor, ln_b: torch.Tensor, eps:
     if H <= 0 or qkv.shape[2] < 3 * H * 64:
         raise ValueError(f"gpa::qk_norm_rope: rows of {qkv.shape[2]} cannot hold q, k, v of "
                          f"{H} heads x 64")
-    w = ln_w.to(device=dev, dtype=torch.float32).contiguous()
-    bb = ln_b.to(device=dev, dtype=torch.float32).contiguous()
-    if w.numel() != 128 or bb.numel() != 128:
-        raise ValueError("gpa::qk_norm_rope: ln_w and ln_b hold the q and k weights, 2 x 64")
     if (pos is None) != (rope_cs is None):
         raise ValueError("gpa::qk_norm_rope: pos and rope_cs go together")
     period, npos = 0, 0
@@ -779,16 +811,20 @@ def qk_norm_rope(qkv: torch.Tensor, ln_w: torch.Tensor, ln_b: torch.Tensor, eps:
     if q.numel() == 0:
         return q, k
     with _on(dev):
-        fn = lib().gpa_qk_norm_rope_f16 if f16 else lib().gpa_qk_norm_rope_bf16
-        rc = fn(
-            qkv.data_ptr(), B, N, H, 64, _st(qkv, 0), _rs(qkv, 1), H * 64,
-            w.data_ptr(), bb.data_ptr(), float(eps),
+        rc = lib().gpa_qk_norm_rope_params(
+            half_code, qkv.data_ptr(), B, N, H, 64, _st(qkv, 0), _rs(qkv, 1), H * 64,
+            *(p.data_ptr() for p in params), _DTYPE_CODES[params[0].dtype], float(eps),
             pos.data_ptr() if pos is not None else None, period,
             rope_cs.data_ptr() if rope_cs is not None else None, npos,
             q.data_ptr(), GPA_DTYPE_F32 if q_f32 else half_code,
             k.data_ptr(), GPA_DTYPE_F32 if k_f32 else half_code, _stream(dev))
     _check(rc, "gpa::qk_norm_rope")
     return q, k
+
+
+@_fake("qk_norm_rope_params")
+def _qk_norm_rope_params_fake(qkv, q_w, k_w, q_b, k_b, eps, pos, rope_cs, heads, q_f32, k_f32):
+    return _qk_norm_rope_fake(qkv, None, None, eps, pos, rope_cs, heads, q_f32, k_f32)
 
 
 @_fake("qk_norm_rope")

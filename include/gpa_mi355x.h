@@ -58,7 +58,7 @@
 extern "C" {
 #endif
 
-#define GPA_ABI_VERSION 17
+#define GPA_ABI_VERSION 18
 
 enum {
   GPA_OK = 0,
@@ -364,6 +364,18 @@ int gpa_qk_norm_rope_f16(const void* qkv, int64_t B, int64_t N, int64_t H, int64
                          const int32_t* pos, int64_t period,
                          const float* rope_cs, int64_t npos,
                          void* q_out, int q_dtype, void* k_out, int k_dtype, void* stream);
+
+/* Either of them (dtype GPA_DTYPE_BF16 or GPA_DTYPE_F16) with the four
+ * LayerNorm parameters of 64 values each where the model holds them, in
+ * param_dtype: GPA_DTYPE_F32, or GPA_DTYPE_BF16 / GPA_DTYPE_F16 16-byte
+ * aligned. */
+int gpa_qk_norm_rope_params(int dtype, const void* qkv, int64_t B, int64_t N, int64_t H,
+                            int64_t D, int64_t qkv_sb, int64_t qkv_sn, int64_t k_offset,
+                            const void* q_weight, const void* k_weight, const void* q_bias,
+                            const void* k_bias, int param_dtype, float eps,
+                            const int32_t* pos, int64_t period, const float* rope_cs,
+                            int64_t npos, void* q_out, int q_dtype, void* k_out, int k_dtype,
+                            void* stream);
 
 /*
  * Pooled summaries of the frame-special shared K/V set.  For every
