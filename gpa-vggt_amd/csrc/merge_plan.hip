@@ -23,14 +23,17 @@
 //
 // What bounds it: launches and latency, not bytes (137,400 tokens are 2 MB).
 // As torch operations this took over 60 launches per merge, three of them
-// merge sorts of up to 16 launches.  Up to kSmall source rows one workgroup
-// per batch element does all of it in LDS, in one launch; above, each pass is
-// two launches over kTile-row blocks (counts per block, then a scatter in
-// which every block sums the counts of the blocks before it; that sum is ~50
-// rows of 1 KB at 200 frames, cheaper than a third launch).  Measured, a
-// whole merge with its K and V: 521 -> 169 us at 4 frames (70 -> 8 launches),
-// 1,394 -> 1,085 us at 100 frames (83 -> 21 launches; the order 5.5 us, the
-// plan ~115 us of the GPU's time), the aggregator on 6 frames 40.0 -> 33.8 ms.
+// merge sorts of up to 16 launches.  Up to kRankMax source rows both orders
+// come from counting: a row's rank is the number of rows before it, ns
+// compares per row spread over the whole chip, one launch for each order.
+// Above, each radix pass is two launches over kTile-row blocks (counts per
+// block, then a scatter in which every block sums the counts of the blocks
+// before it; that sum is ~50 rows of 1 KB at 200 frames, cheaper than a third
+// launch).
+// Measured, a whole merge with its K and V against the torch operations: 521
+// -> 169 us at 4 frames (70 -> 8 launches) with the plan's 38 us in one
+// workgroup, 12 us by counting since; 1,394 -> 1,085 us at 100 frames (83 ->
+// 21 launches; the order 5.5 us, the plan ~115 us of the GPU's time).
 #include "gpa_common.h"
 
 namespace gpa {
@@ -156,10 +159,10 @@ __device__ __forceinline__ int lower_bound(const uint32_t* keys, int n, uint32_t
   return lo;
 }
 
-// Destination slot j's list head, offset and size from the sorted keys.
-__device__ __forceinline__ void place_dst(const PlanArgs& a, int64_t b, int j, const uint32_t* keys) {
+// Destination slot j's list head, offset and size: lo merged rows have a
+// smaller destination, up one no larger.
+__device__ __forceinline__ void place_dst(const PlanArgs& a, int64_t b, int j, int lo, int up) {
   const int unm = a.ns - a.r;
-  const int lo = lower_bound(keys, a.r, j), up = lo + lower_bound(keys + lo, a.r - lo, j + 1);
   const int64_t slot = b * (unm + a.num_dst) + unm + j, off = b * a.N + unm + j + lo;
   a.size[slot] = (float)(1 + up - lo);
   a.offsets[slot] = off;
@@ -223,76 +226,117 @@ __device__ __forceinline__ uint32_t scan_digits(uint32_t x, uint32_t* part) {
   return base + sum - x;
 }
 
-// Up to kSmall source rows: one workgroup per batch element, everything in
-// LDS.  8,192 rows are 8 frames; the LDS (80 KB) and the eight items per
-// thread set the line.  At 4 frames (3,135 rows) the plan takes 38 us here (50
-// with all eight items walked); the 12 to 14 launches of the other path take
-// 4 us each and more.
-constexpr int kSmallThreads = 1024, kSmallItems = 8, kSmall = kSmallThreads * kSmallItems;
+// Ranks by counting.  A workgroup takes 16 rows (or destinations): thread
+// (part, row) compares its row with every 16th group of four keys, staged in
+// LDS kRankKeys at a time, and the 16 parts' counts meet in LDS.  Keys past
+// the end are larger than any that is compared with them.
+constexpr int kRankRows = 16, kRankParts = 16, kRankThreads = kRankRows * kRankParts;
+constexpr int kRankKeys = 4096;
+// Where the two ways cross: the plan at 13,585 source rows takes 67 us by
+// counting and 84 us by radix passes, at 19,855 115 and 86 us (1,045: 8 and
+// 51 us; 3,135: 12 and 65 us; 7,315: 26 and 78 us).
+constexpr int kRankMax = 15360;
+
+// The sum over the parts of each row's counts, for the threads of part 0.
+__device__ __forceinline__ int sum_parts(int x, int (&part)[kRankParts][kRankRows + 1]) {
+  const int r = threadIdx.x % kRankRows;
+  __syncthreads();
+  part[threadIdx.x / kRankRows][r] = x;
+  __syncthreads();
+  int sum = 0;
+#pragma unroll
+  for (int p = 0; p < kRankParts; ++p) sum += part[p][r];
+  return sum;
+}
+
+// Keys base .. base + n of `key` into LDS, the last group of four filled up;
+// all loads first (one at a time, their latency was most of the kernel).
+template <typename Key>
+__device__ __forceinline__ void stage_keys(Key key, int base, int n, uint32_t (&keys)[kRankKeys]) {
+  constexpr int kLoads = kRankKeys / kRankThreads;
+  uint32_t k[kLoads];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int t = u * kRankThreads + threadIdx.x;
+    k[u] = key(base + min(t, n - 1));
+  }
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int t = u * kRankThreads + threadIdx.x;
+    keys[t] = t < n ? k[u] : 0xffffffffu;
+  }
+  __syncthreads();
+}
+
+// Rows before row i = i0 + r in the order of (key, row), over all parts; key(j)
+// gives row j's key, mine is row i's.
+template <typename Key>
+__device__ __forceinline__ int rank_of(Key key, int ns, int i0, uint32_t mine,
+                                       uint32_t (&keys)[kRankKeys],
+                                       int (&part)[kRankParts][kRankRows + 1]) {
+  const int tid = threadIdx.x, r = tid % kRankRows, p = tid / kRankRows;
+  int before = 0;
+  for (int base = 0; base < ns; base += kRankKeys) {
+    const int n = min(kRankKeys, ns - base), n4 = (n + 3) / 4;
+    stage_keys(key, base, n, keys);
+#pragma unroll 4
+    for (int g = p; g < n4; g += kRankParts) {
+      const u32x4 k = *reinterpret_cast<const u32x4*>(&keys[4 * g]);
+      const int j = base + 4 * g;
+      // A tie goes to the earlier row; the workgroup's own rows come below.
+      const uint32_t bound = j < i0 ? mine + 1 : j < i0 + kRankRows ? 0u : mine;
+      before += (k[0] < bound) + (k[1] < bound) + (k[2] < bound) + (k[3] < bound);
+    }
+  }
+  if (i0 + p < ns) before += key(i0 + p) < mine + (p < r ? 1u : 0u);
+  return sum_parts(before, part);
+}
 
 template <typename T>
-__global__ __launch_bounds__(kSmallThreads) void plan_small_kernel(PlanArgs a) {
-  constexpr int kW = kSmallThreads / 64;
-  __shared__ uint32_t keys[kSmall], vals[kSmall];
-  __shared__ uint32_t cnt[kW][kDigits];
-  __shared__ uint32_t base[kDigits], part[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t b = blockIdx.x;
-  const int ns = a.ns, items = (ns + kSmallThreads - 1) / kSmallThreads;   // per thread, <= 8
+__global__ __launch_bounds__(kRankThreads) void rank_rows_kernel(PlanArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t keys[kRankKeys];
+  __shared__ int part[kRankParts][kRankRows + 1];
+  const int64_t b = blockIdx.y;
+  const int i0 = blockIdx.x * kRankRows, i = i0 + threadIdx.x % kRankRows;
+  auto key = [&](int j) { return max_key<T>(a.node_max, b * a.ns + j); };
+  const int rank = rank_of(key, a.ns, i0, i < a.ns ? key(i) : 0u, keys, part);
+  if (threadIdx.x < kRankRows && i < a.ns) a.keys0[b * a.ns + i] = place_rank(a, b, rank, i);
+}
 
-  // One stable pass over (keys, vals) by the digit at `shift`.
-  auto pass = [&](int shift) {
-    uint32_t k[kSmallItems], v[kSmallItems], digit[kSmallItems], rank[kSmallItems];
-    bool live[kSmallItems];
+__global__ __launch_bounds__(kRankThreads) void rank_lists_kernel(PlanArgs a, int row_blocks) {
+  __shared__ __attribute__((aligned(16))) uint32_t keys[kRankKeys];
+  __shared__ int part[kRankParts][kRankRows + 1];
+  const int64_t b = blockIdx.y;
+  const int tid = threadIdx.x, r = tid % kRankRows, p = tid / kRankRows;
+  const uint32_t* const in = a.keys0 + b * a.ns;
+  if ((int)blockIdx.x < row_blocks) {          // source rows
+    const int i0 = blockIdx.x * kRankRows, i = i0 + r;
+    const uint32_t mine = i < a.ns ? in[i] : 0u;
+    const int rank = rank_of([&](int j) { return in[j]; }, a.ns, i0, mine, keys, part);
+    if (p == 0 && i < a.ns && mine < (uint32_t)a.num_dst) place_member(a, b, rank, mine, i);
+    return;
+  }
+  const int j = (blockIdx.x - row_blocks) * kRankRows + r;    // destinations
+  int less = 0, upto = 0;
+  for (int base = 0; base < a.ns; base += kRankKeys) {
+    const int n = min(kRankKeys, a.ns - base), n4 = (n + 3) / 4;
+    stage_keys([&](int j) { return in[j]; }, base, n, keys);
+#pragma unroll 4
+    for (int g = p; g < n4; g += kRankParts) {
+      const u32x4 k = *reinterpret_cast<const u32x4*>(&keys[4 * g]);
 #pragma unroll
-    for (int u = 0; u < kSmallItems; ++u) {
-      const int i = (wave * items + u) * 64 + lane;
-      live[u] = u < items && i < ns;
-      k[u] = live[u] ? keys[i] : 0;
-      v[u] = live[u] ? vals[i] : 0;
-      digit[u] = (k[u] >> shift) & (kDigits - 1);
-    }
-    wave_rank<kSmallItems>(digit, live, items, cnt[wave], rank);
-    __syncthreads();
-    uint32_t total = 0;
-    if (tid < kDigits) {
-#pragma unroll
-      for (int w = 0; w < kW; ++w) {
-        const uint32_t c = cnt[w][tid];
-        cnt[w][tid] = total;
-        total += c;
+      for (int e = 0; e < 4; ++e) {
+        less += k[e] < (uint32_t)j;
+        upto += k[e] <= (uint32_t)j;
       }
     }
-    const uint32_t first = scan_digits(total, part);
-    if (tid < kDigits) base[tid] = first;
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kSmallItems; ++u)
-      if (live[u]) {
-        const uint32_t to = base[digit[u]] + cnt[wave][digit[u]] + rank[u];
-        keys[to] = k[u];
-        vals[to] = v[u];
-      }
-    __syncthreads();
-  };
-
-  for (int i = tid; i < ns; i += kSmallThreads) {
-    keys[i] = max_key<T>(a.node_max, b * ns + i);
-    vals[i] = i;
   }
-  __syncthreads();
-  for (int p = 0; p < 4; ++p) pass(8 * p);
-  for (int i = tid; i < ns; i += kSmallThreads) {
-    const uint32_t e = vals[i];
-    keys[e] = place_rank(a, b, i, e);
-  }
-  __syncthreads();
-  for (int i = tid; i < ns; i += kSmallThreads) vals[i] = i;
-  __syncthreads();
-  for (int p = 0; p < a.passes; ++p) pass(8 * p);
-  for (int j = tid; j < a.num_dst; j += kSmallThreads) place_dst(a, b, j, keys);
-  for (int i = tid; i < a.r; i += kSmallThreads) place_member(a, b, i, keys[i], vals[i]);
-  if (b == a.B - 1 && tid == 0) a.offsets[a.B * (int64_t)(ns - a.r + a.num_dst)] = a.B * a.N;
+  less = sum_parts(less, part);
+  upto = sum_parts(upto, part);
+  if (p == 0 && j < a.num_dst) place_dst(a, b, j, less, upto);
+  if (blockIdx.x == gridDim.x - 1 && b == a.B - 1 && tid == 0)
+    a.offsets[a.B * (int64_t)(a.ns - a.r + a.num_dst)] = a.B * a.N;
 }
 
 // More rows: kTile rows per block, grid (blocks, B).
@@ -396,20 +440,32 @@ __global__ __launch_bounds__(kPlaceThreads) void plan_lists_kernel(PlanArgs a, c
                                                                    const uint32_t* rows) {
   const int64_t b = blockIdx.y;
   const int i = blockIdx.x * kPlaceThreads + threadIdx.x;
-  if (i < a.num_dst) place_dst(a, b, i, keys + b * a.ns);
+  if (i < a.num_dst) {
+    const uint32_t* k = keys + b * a.ns;
+    const int lo = lower_bound(k, a.r, i);
+    place_dst(a, b, i, lo, lo + lower_bound(k + lo, a.r - lo, i + 1));
+  }
   if (i < a.r) place_member(a, b, i, keys[b * a.ns + i], rows[b * a.ns + i]);
   if (i == 0 && b == a.B - 1) a.offsets[a.B * (int64_t)(a.ns - a.r + a.num_dst)] = a.B * a.N;
 }
 
 size_t plan_ws_bytes(int64_t B, int64_t ns) {
-  if (ns <= kSmall) return 0;
+  if (ns <= kRankMax) return (size_t)B * ns * sizeof(uint32_t);
   return (size_t)B * (4 * ns + (ns + kTile - 1) / kTile * kDigits) * sizeof(uint32_t);
 }
 
 template <typename T>
 void plan_launch(const PlanArgs& a, hipStream_t s) {
-  if (a.ns <= kSmall) {
-    hipLaunchKernelGGL(plan_small_kernel<T>, dim3((unsigned)a.B), dim3(kSmallThreads), 0, s, a);
+  if (a.ns <= kRankMax) {
+    const int row_blocks = (a.ns + kRankRows - 1) / kRankRows;
+    const int dst_blocks = (a.num_dst + kRankRows - 1) / kRankRows;
+    if (a.ns > 0)
+      hipLaunchKernelGGL(rank_rows_kernel<T>, dim3((unsigned)row_blocks, (unsigned)a.B),
+                         dim3(kRankThreads), 0, s, a);
+    // At least one destination block: the last one closes the offsets.
+    hipLaunchKernelGGL(rank_lists_kernel,
+                       dim3((unsigned)(row_blocks + (dst_blocks > 0 ? dst_blocks : 1)), (unsigned)a.B),
+                       dim3(kRankThreads), 0, s, a, row_blocks);
     return;
   }
   const dim3 grid((unsigned)a.blocks, (unsigned)a.B), block(kSortThreads);
@@ -561,8 +617,8 @@ extern "C" int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t
   a.passes = 1;
   while (a.passes < 4 && (top >> (8 * a.passes)) != 0) ++a.passes;
   a.blocks = (int)((ns + kTile - 1) / kTile);
-  if (need) {
-    a.keys0 = (uint32_t*)workspace;
+  a.keys0 = (uint32_t*)workspace;
+  if (ns > kRankMax) {
     a.keys1 = a.keys0 + B * ns;
     a.vals0 = a.keys1 + B * ns;
     a.vals1 = a.vals0 + B * ns;

@@ -1,6 +1,7 @@
 """The merge's bookkeeping kernels (gpa::merge_order, gpa::merge_plan) against
 torch's stable sorts: exact, every output.  Row counts sit at the edges of the
-one-workgroup path (8,192 rows) and of the radix sort's blocks (4,096 rows);
+counting path (up to 15,360 rows; 16 rows a workgroup, 4,096 keys staged at a
+time) and of the radix sort's blocks (4,096 rows);
 maxima with ties, NaN, both zeros and infinities; all rows of a batch element
 in one slot; destination counts of one to three key bytes."""
 import pytest
@@ -48,7 +49,8 @@ def _expected(node_max, node_idx, order, num_dst, r):
     return edge, dst_slot, unm_abs, src_abs, size, offsets, tokens
 
 
-@pytest.mark.parametrize("ns", [0, 1, 64, 1023, 1045, 8191, 8192, 8193, 12288, 20481])
+@pytest.mark.parametrize("ns", [0, 1, 15, 64, 1023, 1045, 4096, 4097, 8193, 15360, 15361,
+                                20481])
 @pytest.mark.parametrize("num_dst,share,dtype,kind", [
     (1, 1.0, torch.float32, "plain"), (255, 0.2, torch.float32, "ties"),
     (256, 1.0, torch.bfloat16, "special"), (300, 0.0, torch.float16, "ties"),
