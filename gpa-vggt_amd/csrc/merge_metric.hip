@@ -97,13 +97,21 @@ __global__ __launch_bounds__(kThreads, 1) void merge_metric_kernel(MetricArgs a)
     asm volatile("" : "+v"(bfrag[ks]));
   }
 
-  auto load = [&](Raw (&raw)[kLoads], int blk) {
+  // The row of a block step, its index fetched two steps before its loads are
+  // issued, so that these never wait for it (137,400 bf16 rows of 1,024: 94.3
+  // -> 91.6 us).
+  struct Row {
+    int64_t b, t;
+  };
+  auto row_of = [&](int blk) {
     int64_t i = (int64_t)blk * kRows + lr;
     if (i >= a.rows) i = a.rows - 1;                     // tail rows: any valid row
-    const int64_t b = i / a.N, j = i - b * a.N;
-    const int64_t t = a.order ? a.order[j] : j;
+    const int64_t b = a.rows == a.N ? 0 : i / a.N, j = i - b * a.N;
+    return Row{b, a.order ? a.order[j] : j};
+  };
+  auto load = [&](Raw (&raw)[kLoads], const Row& at) {
     const Raw* row = reinterpret_cast<const Raw*>(
-        static_cast<const char*>(a.x) + (b * a.sb + t * a.sn) * (F32 ? 4 : 2));
+        static_cast<const char*>(a.x) + (at.b * a.sb + at.t * a.sn) * (F32 ? 4 : 2));
 #pragma unroll
     for (int l = 0; l < kLoads; ++l) raw[l] = row[l * 32 + lc];
   };
@@ -169,15 +177,20 @@ __global__ __launch_bounds__(kThreads, 1) void merge_metric_kernel(MetricArgs a)
   const int G = gridDim.x;
   int blk = blockIdx.x;
   Raw raw0[kLoads], raw1[kLoads];
-  load(raw0, blk);
-  load(raw1, blk + G);
+  Row at0 = row_of(blk), at1 = row_of(blk + G);
+  load(raw0, at0);
+  load(raw1, at1);
+  at0 = row_of(blk + 2 * G);
+  at1 = row_of(blk + 3 * G);
   for (; blk < a.nblocks; blk += 2 * G) {
     stage(raw0);
-    load(raw0, blk + 2 * G);
+    load(raw0, at0);
+    at0 = row_of(blk + 4 * G);
     finish(blk);
     if (blk + G >= a.nblocks) break;                     // workgroup-uniform
     stage(raw1);
-    load(raw1, blk + 3 * G);
+    load(raw1, at1);
+    at1 = row_of(blk + 5 * G);
     finish(blk + G);
   }
 }
