@@ -1,0 +1,44 @@
+"""Head dim 64 on both sides of the line where the attention forms its row
+bounds itself (8,192 keys): certified, tile-0 and lazily moved offsets (logit
+scales from 0.3 to 30), an outlier key in the first and in the last tile.
+
+Bar: a row's relative error within 16-bit P and output, 4 * 2^-9 (bf16) or
+4 * 2^-12 (fp16) of unit-scale values."""
+import pytest
+import torch
+
+from merging import _native
+from merging.fused_attention import attention_keybias
+from oracle.attention import attention_reference
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N", [8160, 8192, 8193])
+@pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -9), (torch.float16, 2.0 ** -12)])
+@pytest.mark.parametrize("scale,outlier", [(0.3, None), (3.0, None), (0.5, 0), (0.5, -1)])
+def test_bounds_formed_in_the_kernel(dev, N, dtype, ulp, scale, outlier):
+    g = torch.Generator().manual_seed(N)
+    q = (torch.randn(1, 2, 130, 64, generator=g) * scale).to(dtype)
+    k = torch.randn(1, 2, N, 64, generator=g) * scale
+    if outlier is not None:
+        k[:, :, outlier] *= 12.0
+    k, v = k.to(dtype), torch.randn(1, 2, N, 64, generator=g).to(dtype)
+    bias = torch.randint(1, 9, (1, 1, 1, N), generator=g).float().log().expand(1, 2, 1, N).to(dtype)
+    o = attention_keybias(q.to(dev), k.to(dev), v.to(dev), bias.to(dev), 0.125)
+    ref, _ = attention_reference(q, k, v, bias, 0.125)
+    rel = (o.float().cpu() - ref).norm(dim=-1) / ref.norm(dim=-1)
+    assert rel.max().item() <= 4 * ulp, rel.max().item()
+
+
+def test_certified_on_both_sides(dev):
+    """The same keys, one more at -inf: the same bound, the same offset."""
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(1, 1, t, 64, generator=g).mul(0.5).bfloat16().to(dev)
+               for t in (200, 8193, 8193))
+    bias = torch.zeros(1, 1, 1, 8193, device=dev)
+    bias[..., 8192] = float("-inf")
+    _, _, few = _native.attn_keybias_offset_flags(q, k[:, :, :8192], v[:, :, :8192],
+                                                  bias[..., :8192], 0.125)
+    _, _, more = _native.attn_keybias_offset_flags(q, k, v, bias, 0.125)
+    assert not few.any() and not more.any()
