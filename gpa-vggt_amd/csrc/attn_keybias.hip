@@ -351,12 +351,11 @@ __device__ __forceinline__ void tile_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Tile records of a call without bias, bf16 (the own-frame and frame
-// attentions): bias/sm_scale = 0 for the keys, -inf past N, and no key
+// Tile records of a joined call without bias, bf16 (unjoined ones need none:
+// attn_plain_kernel): bias/sm_scale = 0 for the keys, -inf past N, and no key
 // maxima, so the kernel has no score bound and every wave takes the tile-0
 // offset or the lazily moved one.  Writing these costs nothing like reading
-// every key (tile_records_kernel reads all of K: 0.11 of the own-frame
-// call's 1.86 ms).  Also zeroes the row-bound words the kernel reads.
+// every key.  Also zeroes the row-bound words the kernel reads.
 __global__ __launch_bounds__(256) void fill_records_kernel(float* recs, float* bounds,
                                                            int64_t ntiles, int64_t N,
                                                            int64_t total, int64_t rows) {
@@ -427,7 +426,21 @@ struct alignas(16) MainTile {
   float rec[64];
 };
 
-template <bool F16, bool JOIN>
+// Records of a call without bias are zeros, but for the keys past N of the last
+// tile: row N % 32 of this table, -inf from there on (row 0: a whole tile).
+struct TailRecords {
+  float w[kKT][kRec];
+};
+constexpr TailRecords tail_records() {
+  TailRecords t{};
+  for (int r = 1; r < kKT; ++r)
+    for (int k = r; k < kKT; ++k) t.w[r][k] = -__builtin_inff();
+  return t;
+}
+__device__ const TailRecords kTail = tail_records();
+
+// PLAIN: no bias and no score bound (bf16), so no records in memory.
+template <bool F16, bool JOIN, bool PLAIN>
 __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
   __shared__ MainTile ring0, ring1, ring2, ring3, ring4;
   __shared__ float rec_sink[64];
@@ -456,7 +469,7 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
   const uint16_t* Q = p.q + b * p.q_sb + h * p.q_sh;
   const uint16_t* K = p.k + b * p.k_sb + h * p.k_sh;
   const uint16_t* V = p.v + b * p.v_sb + h * p.v_sh;
-  const float* R = p.recs + (int64_t)bh * (p.rec_bytes / 4);
+  const float* R = PLAIN ? kTail.w[(int)p.N & (kKT - 1)] : p.recs + (int64_t)bh * (p.rec_bytes / 4);
   // The output bases, formed here so that only two pointers (not five
   // 64-bit strides) stay live in SGPRs until the epilogue.
   uint16_t* O = p.o + b * p.o_sb + h * p.o_sh;
@@ -466,8 +479,9 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
   else asm volatile("" : "+s"(O), "+s"(LSE));
 
   const float* const rb = p.bounds + (int64_t)kBoundWords * bh;
-  float row_k, row_b, row_kmean, row_bmean;
-  if (p.fold) {
+  float row_k = 0.f, row_b = 0.f, row_kmean = 0.f, row_bmean = 0.f;
+  if constexpr (PLAIN) {
+  } else if (p.fold) {
     const int nt = (int)((p.N + kKT - 1) / kKT);
     float kb = 0.f, bb = -INFINITY, ks = 0.f, bs = 0.f;
     u32x2 w2[kFoldLoads];
@@ -525,7 +539,7 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
 
   const __amdgpu_buffer_rsrc_t krs = make_rsrc(K, p.k_bytes);
   const __amdgpu_buffer_rsrc_t vrs = make_rsrc(V, p.v_bytes);
-  const __amdgpu_buffer_rsrc_t rrs = make_rsrc(R, p.rec_bytes);
+  const __amdgpu_buffer_rsrc_t rrs = make_rsrc(R, PLAIN ? kRec * 4u : p.rec_bytes);
   const uint32_t k_row = (uint32_t)p.k_sn * 2u, v_row = (uint32_t)p.v_sn * 2u;
   const int slot = wave * 64 + lane;
   const int s_key = slot >> 3, s_pc = slot & 7;
@@ -541,7 +555,10 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
     dma16(krs, &T.k[wave * 512], k_voff, n0 * k_row);
     dma16(vrs, &T.v[wave * 512], v_voff, n0 * v_row);
     float* dst = wave == 0 ? &T.rec[0] : &rec_sink[0];   // wave-uniform M0, no branch
-    dma4(rrs, dst, rec_voff, (uint32_t)t * (kRec * 4));
+    if constexpr (PLAIN)       // every tile but the last lands zeros: an empty range
+      dma4(make_rsrc(R, t == ntiles - 1 ? kRec * 4u : 0u), dst, rec_voff, 0);
+    else
+      dma4(rrs, dst, rec_voff, (uint32_t)t * (kRec * 4));
   };
   // A tile has landed once at most the DMAs of the NT tiles issued after it
   // (three instructions per tile) are outstanding.
@@ -742,7 +759,7 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
     bad = bad || !(x0s[j] >= m_off[j] - kDown<F16>);     // NaN scores fail too
   }
   // (Without the key maxima there is no bound to certify anything with.)
-  fixed = !p.no_bound && __builtin_amdgcn_ballot_w64(bad) == 0;
+  fixed = !PLAIN && !p.no_bound && __builtin_amdgcn_ballot_w64(bad) == 0;
   float lo[kBlk], outl[kBlk];
   if (!fixed) {
     // The tile-0 offset, taken where tile 0's scores are narrow and no key
@@ -1049,7 +1066,15 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
 
 template <bool F16>
 __global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
-  attn_main_body<F16, false>(p);
+  attn_main_body<F16, false, false>(p);
+}
+
+// bf16 attention without bias (the frame and own-frame attentions): one launch
+// where filling the records was another.  16 heads, 1,374 queries and keys per
+// frame: 1 frame 29.0 -> 27.0 us, 4 frames 45.4 -> 43.1, 16 frames 135.5 ->
+// 131.6, 100 frames (own keys) 854 -> 845.
+__global__ __launch_bounds__(kThreads, 2) void attn_plain_kernel(AttnArgs p) {
+  attn_main_body<false, false, true>(p);
 }
 
 // The second attention of a split key set, joined with the first in its
@@ -1059,7 +1084,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_main_kernel(AttnArgs p) {
 // from 569 to 524 us).
 template <bool F16>
 __global__ __launch_bounds__(kThreads, 2) void attn_join_kernel(AttnJoinArgs p) {
-  attn_main_body<F16, true>(p.a);
+  attn_main_body<F16, true, false>(p.a);
 }
 
 // Workspace: one row of ntiles tile records per (batch, head), then
@@ -1235,7 +1260,9 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
   ra.total = B * H * ntiles;
   float* bounds = (float*)((char*)workspace + rec_bytes(B, H, N));
   const bool no_bound = bias_kind == GPA_BIAS_NONE && !F16;
-  if (no_bound) {
+  const bool plain = no_bound && !join;
+  if (plain) {
+  } else if (no_bound) {
     const int64_t n = ra.total * kRec;
     hipLaunchKernelGGL(fill_records_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
                        (float*)workspace, bounds, ntiles, N, ra.total, B * H);
@@ -1302,6 +1329,8 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
   const dim3 grid((unsigned)gx, (unsigned)(B * H)), block(kThreads);
   if (join)
     hipLaunchKernelGGL(attn_join_kernel<F16>, grid, block, 0, s, AttnJoinArgs{p, *join});
+  else if (plain)
+    hipLaunchKernelGGL(attn_plain_kernel, grid, block, 0, s, p);
   else
     hipLaunchKernelGGL(attn_main_kernel<F16>, grid, block, 0, s, p);
   e = hipGetLastError();
