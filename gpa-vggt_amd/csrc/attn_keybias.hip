@@ -304,9 +304,12 @@ constexpr int kBoundWords = 4;
 // Up to this many tiles (8,192 keys) every wave of the attention forms them
 // from the records itself, which saves the launch: 16 heads, 2,748 queries and
 // 1,703 keys 38.4 -> 36.7 us, 5,496 x 2,361 76.6 -> 75.4 us, 21,984 x 7,721
-// within 0.1 %.  (The records and the bounds by one workgroup per head in one
+// within 0.1 %.  It delays every workgroup a little, though, so the line lies
+// at two rounds of the chip's 512 places: 40 fp16 frames (3,840 workgroups of
+// 43 tiles) took 352 us so and take 348 us with the launch.  (The records and the bounds by one workgroup per head in one
 // launch took 6 us more than the two launches.)
 constexpr int kFoldLoads = 4, kFoldTiles = 64 * kFoldLoads;
+constexpr int64_t kFoldGrid = 1024;
 __global__ __launch_bounds__(256) void row_bounds_kernel(const float* recs, float* bounds,
                                                          int64_t ntiles) {
   __shared__ float part[4][4];
@@ -755,6 +758,9 @@ __device__ __forceinline__ void attn_main_body(const AttnArgs& p) {
 #pragma unroll
   for (int j = 0; j < kBlk; ++j) {
     x0s[j] = row_max(s_cur[j]);
+    // (A value of its own in every kernel, not one end of an FMA with kDown in
+    // the one that has no other use for it: the same offset, the same P.)
+    asm volatile("" : "+v"(x0s[j]));
     m_off[j] = fmaxf(__builtin_fmaf(q_norm[j], row_k, row_b) - kUp<F16>, x0s[j]);
     bad = bad || !(x0s[j] >= m_off[j] - kDown<F16>);     // NaN scores fail too
   }
@@ -1289,7 +1295,7 @@ int attn_keybias_run(const char* fn, const void* q, const void* k, const void* v
                   hipGetErrorString(e));
     return GPA_E_LAUNCH;
   }
-  const bool fold = !no_bound && ntiles <= kFoldTiles;
+  const bool fold = !no_bound && ntiles <= kFoldTiles && gx * B * H <= kFoldGrid;
   if (!no_bound && !fold) {
     hipLaunchKernelGGL(row_bounds_kernel, dim3((unsigned)(B * H)), dim3(256), 0, s,
                        (const float*)workspace, bounds, ntiles);

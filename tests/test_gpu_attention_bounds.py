@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from merging import _native
-from merging.fused_attention import attention_keybias
+from merging.fused_attention import attention_join, attention_keybias
 from oracle.attention import attention_reference
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +42,27 @@ def test_certified_on_both_sides(dev):
                                                   bias[..., :8192], 0.125)
     _, _, more = _native.attn_keybias_offset_flags(q, k, v, bias, 0.125)
     assert not few.any() and not more.any()
+
+
+@pytest.mark.parametrize("N", [1, 2, 31, 32, 33, 47, 64, 95, 128, 129, 159, 160, 161])
+@pytest.mark.parametrize("join", [False, True])
+def test_last_tile_without_bias(dev, N, join):
+    """The last tile's mask of a call without bias, alone and joined: k and v are
+    views of longer buffers whose rows past N hold NaN."""
+    g = torch.Generator().manual_seed(N)
+    q, k, v = (torch.randn(1, 2, t, 64, generator=g).bfloat16() for t in (70, N, N))
+    long = [torch.full((1, 2, N + 200, 64), float("nan"), dtype=q.dtype, device=dev) for _ in "kv"]
+    for buf, t in zip(long, (k, v)):
+        buf[:, :, :N] = t.to(dev)
+    kd, vd = (buf[:, :, :N] for buf in long)
+    ref, ref_lse = attention_reference(q, k, v, None, 0.125)
+    if join:
+        other = torch.zeros(2, 2, 35, 64, dtype=q.dtype, device=dev)
+        o = attention_join(q.to(dev), kd, vd, None, 0.125, other,
+                           torch.full((2, 2, 35), -1e4, device=dev), 2)
+        o = o.view(1, 70, 2, 64).transpose(1, 2)
+    else:
+        o, lse = attention_keybias(q.to(dev), kd, vd, None, 0.125, return_lse=True)
+        assert (lse.cpu() - ref_lse).abs().max().item() <= 2.0 ** -8 / 0.6931   # bf16 P in the sum
+    rel = (o.float().cpu() - ref).norm(dim=-1) / ref.norm(dim=-1)
+    assert rel.max().item() <= 4 * 2.0 ** -9, rel.max().item()
