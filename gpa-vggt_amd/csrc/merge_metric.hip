@@ -97,16 +97,24 @@ __global__ __launch_bounds__(kThreads, 1) void merge_metric_kernel(MetricArgs a)
     asm volatile("" : "+v"(bfrag[ks]));
   }
 
-  // The row of a block step, its index fetched two steps before its loads are
-  // issued, so that these never wait for it (137,400 bf16 rows of 1,024: 94.3
-  // -> 91.6 us).
+  // The row of a block step.  kAhead: its index is fetched two steps before its
+  // loads are issued, so that these never wait for it; otherwise with them.
+  // Ahead costs registers, which the widest fp32 rows do not have: at C = 1024
+  // the fp32 loads then wait on the moves around them, and the fp16 projection
+  // spills.  Microseconds with the loads and ahead, 137,400 rows:
+  //            C = 256        512            768            1024
+  //   bf16     65.0 / 59.5    72.6 / 68.3    79.9 / 75.5    94.4 / 89.9
+  //   fp32     67.5 / 61.3    81.3 / 78.8    112.5 / 107.5  137.1 / 142.8
+  //   to fp16  68.8 / 63.0    83.4 / 84.5    111.5 / 110.1  144.8 / 167.0
+  // (fp16 projection ahead at 256 only: at 768 the two lie within the noise.)
+  constexpr bool kAhead = !F32 || (P16 ? C <= 256 : C <= 768);
   struct Row {
     int64_t b, t;
   };
   auto row_of = [&](int blk) {
     int64_t i = (int64_t)blk * kRows + lr;
     if (i >= a.rows) i = a.rows - 1;                     // tail rows: any valid row
-    const int64_t b = a.rows == a.N ? 0 : i / a.N, j = i - b * a.N;
+    const int64_t b = kAhead && a.rows == a.N ? 0 : i / a.N, j = i - b * a.N;
     return Row{b, a.order ? a.order[j] : j};
   };
   auto load = [&](Raw (&raw)[kLoads], const Row& at) {
@@ -177,20 +185,35 @@ __global__ __launch_bounds__(kThreads, 1) void merge_metric_kernel(MetricArgs a)
   const int G = gridDim.x;
   int blk = blockIdx.x;
   Raw raw0[kLoads], raw1[kLoads];
-  Row at0 = row_of(blk), at1 = row_of(blk + G);
-  load(raw0, at0);
-  load(raw1, at1);
-  at0 = row_of(blk + 2 * G);
-  at1 = row_of(blk + 3 * G);
+  Row at0, at1;
+  if constexpr (kAhead) {
+    at0 = row_of(blk);
+    at1 = row_of(blk + G);
+    load(raw0, at0);
+    load(raw1, at1);
+    at0 = row_of(blk + 2 * G);
+    at1 = row_of(blk + 3 * G);
+  } else {
+    load(raw0, row_of(blk));
+    load(raw1, row_of(blk + G));
+  }
   for (; blk < a.nblocks; blk += 2 * G) {
     stage(raw0);
-    load(raw0, at0);
-    at0 = row_of(blk + 4 * G);
+    if constexpr (kAhead) {
+      load(raw0, at0);
+      at0 = row_of(blk + 4 * G);
+    } else {
+      load(raw0, row_of(blk + 2 * G));
+    }
     finish(blk);
     if (blk + G >= a.nblocks) break;                     // workgroup-uniform
     stage(raw1);
-    load(raw1, at1);
-    at1 = row_of(blk + 5 * G);
+    if constexpr (kAhead) {
+      load(raw1, at1);
+      at1 = row_of(blk + 5 * G);
+    } else {
+      load(raw1, row_of(blk + 3 * G));
+    }
     finish(blk + G);
   }
 }

@@ -210,3 +210,22 @@ def test_token_merge_under_fp16_autocast(dev):
     keep = (bf16_top2_gap(a, b) >= 1e-3).cpu()
     assert keep.float().mean() > 0.5
     assert torch.equal(ix.node_idx.cpu()[keep], ref_idx[keep])
+
+
+@pytest.mark.parametrize("C", [256, 512, 768, 1024])
+@pytest.mark.parametrize("dtype,mode", [(torch.float32, 0), (torch.bfloat16, 0),
+                                        (torch.float32, 2)])
+@pytest.mark.parametrize("N", [15, 4096, 4113, 12_305])
+def test_every_instance_at_the_edges_of_its_steps(dev, C, dtype, mode, N):
+    """Each width and rounding at fewer rows than one block step, at exactly
+    one step of every workgroup (256 of 16 rows), one row more and a step
+    past three: indices fetched ahead of the loads reach past the last row."""
+    g = torch.Generator().manual_seed(C + N)
+    metric = torch.randn(2, N, C, generator=g).to(dev, dtype)
+    proj_f32 = torch.randn(C, 128, generator=g).to(dev)
+    half = torch.float16 if mode == 2 else torch.bfloat16
+    order = torch.randperm(N, generator=g).to(dev)
+    got = _native.merge_metric(metric, proj_f32.to(half), order, mode)
+    chain = _torch_chain(metric, proj_f32, order, True, half)
+    _compare(got, chain, _fp64_chain(metric, proj_f32.to(half), order, False),
+             f"C={C} {dtype} mode {mode} N={N}")

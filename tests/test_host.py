@@ -486,3 +486,16 @@ def test_bench_measures_one_gpu_and_prices_against_the_bf16_peak(capsys):
     assert abs(e["pct_peak"] - 100 * e["tflops"] / 2516.6) < 0.01
     args = bench.parse_args([])
     assert args.gpus == 1 and args.steps > 0 and args.warmup >= 0
+
+
+def test_merge_metric_kernels_have_no_spills_or_scratch():
+    """Every instance of the merge front end keeps its registers: at C = 1024
+    the resident projection leaves so few that holding one more value spills."""
+    import shutil
+    if shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists():
+        pytest.skip("hipcc not available")
+    kernels = _build_module().resource_usage(["merge_metric.hip"])["merge_metric.hip"]
+    assert len(kernels) == 12                  # four widths x (bf16, fp32, fp32 to fp16)
+    bad = {n: u for n, u in kernels.items()
+           if u.get("vgpr_spill") or u.get("sgpr_spill") or u.get("scratch")}
+    assert not bad, f"kernels with spills or scratch: {bad}"
