@@ -67,7 +67,11 @@ __global__ __launch_bounds__(kOrderThreads) void merge_order_kernel(OrderArgs a)
     if (!is_dst && j < drawn) {
       const int64_t y = j / row_len, x = j % row_len;
       const int64_t win = ((int64_t)(f - 1) * a.hsy + y / a.sy) * a.wsx + x / a.sx;
-      is_dst = a.cell[win] == (y % a.sy) * a.sx + x % a.sx;
+      // A cell outside its window counts as the nearest one inside: every window
+      // then has its one destination, and the ranks stay inside `order`.
+      const int64_t drawn_cell = a.cell[win], last = (int64_t)a.sy * a.sx - 1;
+      is_dst = (drawn_cell < 0 ? 0 : drawn_cell > last ? last : drawn_cell) ==
+               (y % a.sy) * a.sx + x % a.sx;
     }
     is_dst = is_dst && p < a.tpi;
     const uint64_t votes = __builtin_amdgcn_ballot_w64(is_dst);

@@ -29,6 +29,29 @@ def test_order_and_mask(dev, frames, w, h, sx, sy, ns, no_rand):
     assert int((mask == -1).sum()) == num_dst_tokens(frames, w, h, sx, sy, ns, no_rand)
 
 
+@pytest.mark.parametrize("bad", [-1, 6, -2 ** 40, 2 ** 40])
+@pytest.mark.parametrize("every", [1, 3])
+def test_cells_outside_their_window(dev, bad, every):
+    """They count as the nearest cell inside, and nothing is written past the
+    mask and the order (a mask without a destination in a window would shift
+    the sources' ranks past the end)."""
+    frames, w, h, sx, sy, ns = 3, 13, 8, 2, 3, 5
+    n, pad = frames * (w * h + ns), 256
+    cell = torch.randint(0, 6, (frames - 1, h // sy, w // sx),
+                         generator=torch.Generator().manual_seed(5))
+    cell.view(-1)[::every] = bad
+    want_mask, want = torch.ops.gpa.merge_order(cell.clamp(0, 5).to(dev), frames, w, h, sx, sy, ns,
+                                                dev)
+    mask, order = (torch.full((n + pad,), -7, device=dev, dtype=torch.int64) for _ in range(2))
+    cell = cell.to(dev)
+    rc = _native.lib().gpa_merge_order(cell.data_ptr(), frames, w, h, sx, sy, ns, mask.data_ptr(),
+                                       order.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == _native.GPA_OK
+    assert torch.equal(mask[:n], want_mask) and torch.equal(order[:n], want)
+    assert (mask[n:] == -7).all() and (order[n:] == -7).all()
+    assert torch.equal(want, torch.argsort(want_mask, stable=True))
+
+
 def _expected(node_max, node_idx, order, num_dst, r):
     """The same lists from torch's stable sorts, on the CPU."""
     B, ns = node_max.shape
