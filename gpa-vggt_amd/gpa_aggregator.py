@@ -454,13 +454,21 @@ class Block(nn.Module):
         return x + self.ls2(self.mlp(self.norm2(x))), None
 
 
+_MODULE_CALL, _BLOCK_FORWARD = nn.Module.__call__, Block.forward
+
+
 def _chainable(blk: nn.Module) -> bool:
-    """A plain Block whose call does no more than its `step`: no hooks, no
-    replaced forward."""
+    """A plain Block whose call would do no more than its `step`: no forward or
+    backward hook of its own or of all modules, not compiled, not traced,
+    neither its forward nor the call itself replaced."""
     mod = torch.nn.modules.module
-    return (type(blk) is Block and "forward" not in blk.__dict__ and not blk._forward_hooks
-            and not blk._forward_pre_hooks and not mod._global_forward_hooks
-            and not mod._global_forward_pre_hooks)
+    return (type(blk) is Block and Block.__call__ is _MODULE_CALL
+            and Block.forward is _BLOCK_FORWARD and "forward" not in blk.__dict__
+            and blk._compiled_call_impl is None and torch._C._get_tracing_state() is None
+            and not (blk._forward_hooks or blk._forward_pre_hooks or blk._backward_hooks
+                     or blk._backward_pre_hooks or mod._global_forward_hooks
+                     or mod._global_forward_pre_hooks or mod._global_backward_hooks
+                     or mod._global_backward_pre_hooks))
 
 
 def _chain_step(blk, x, ln1, rope=None, global_merging=None, following=None):
