@@ -471,13 +471,14 @@ def _chainable(blk: nn.Module) -> bool:
                      or mod._global_backward_pre_hooks))
 
 
-def _chain_step(blk, x, ln1, rope=None, global_merging=None, following=None):
-    """One block of a chain: `Block.step`, or the module call where something
-    hangs on it (and then without the LayerNorms shared between blocks)."""
+def _chain_step(blk, x, ln1, *args, following=None):
+    """One block of a chain, called with (x, *args): `Block.step`, or the module
+    call where something hangs on it or another module takes the block's place
+    (and then without the LayerNorms shared between blocks)."""
     if not _chainable(blk):
-        return blk(x, rope, global_merging), None
-    return blk.step(x, ln1, rope, global_merging,
-                    following if following is not None and _chainable(following) else None)
+        return blk(x, *args), None
+    return blk.step(x, ln1, *args,
+                    following=following if following is not None and _chainable(following) else None)
 
 
 class DinoV2Reg(nn.Module):

@@ -95,3 +95,41 @@ def test_tracers_record_the_blocks(vit):
     assert called == ["blocks.0", "blocks.1", "blocks.2", "norm"]
     graph = str(torch.jit.trace(vit, _image(), check_trace=False).graph)
     assert graph.count("prim::CallMethod") == 4            # the same modules
+
+
+def test_other_modules_in_a_block_s_place(vit):
+    """They are called with what the loop passes, the image tokens alone."""
+    img, args = _image(), []
+    base = vit(img)
+    handle = vit.blocks[1].register_forward_pre_hook(lambda m, a: args.append(len(a)))
+    assert torch.equal(vit(img), base) and args == [1]
+    handle.remove()
+    vit.blocks[1] = torch.nn.Sequential(vit.blocks[1])
+    assert torch.equal(vit(img), base)
+    vit.blocks[1] = torch.nn.Identity()
+    assert vit(img).shape == base.shape
+
+
+def test_arguments_of_the_aggregator_s_blocks():
+    cfg = A.GpaConfig(img_size=84, vit_depth=1, depth=2, embed_dim=64, num_heads=2)
+    model, seen = A.GpaAggregator(cfg), []
+
+    class Record(torch.nn.Module):
+        def __init__(self, name):
+            super().__init__()
+            self.name = name
+
+        def forward(self, x, *args):
+            seen.append((self.name, len(args)))
+            return x
+
+    class Embed(torch.nn.Module):
+        def forward(self, images):
+            return torch.zeros(images.shape[0], 36, 64)
+
+    model.patch_embed = Embed()
+    for i in range(cfg.depth):
+        model.frame_blocks[i], model.global_blocks[i] = Record("frame"), Record("global")
+    with torch.no_grad():
+        model(torch.zeros(1, 2, 3, 84, 84))
+    assert seen == [("frame", 1), ("global", 2)] * cfg.depth
