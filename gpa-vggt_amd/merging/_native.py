@@ -310,12 +310,13 @@ def _op(fn):
     torch.library.register_autograd(f"gpa::{name}", backward, lib=_LIB)
     op = getattr(torch.ops.gpa, name).default
 
-    def call(*args):
+    def call(*args, **kwargs):
         if torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
-                isinstance(a, torch.Tensor) and a.requires_grad for a in args)):
-            return op(*args)
+                isinstance(a, torch.Tensor) and a.requires_grad
+                for a in (*args, *kwargs.values()))):
+            return op(*args, **kwargs)
         with _Below():
-            return op(*args)
+            return op(*args, **kwargs)
 
     call.__name__, call.__doc__ = name, fn.__doc__
     return call

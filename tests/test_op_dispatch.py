@@ -48,3 +48,16 @@ def test_cpu_tensors_are_refused():
     q = torch.zeros(1, 1, 4, 64, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU tensors"):
         _native.attn_keybias(q, q, q, None, 0.125, False)
+
+
+def test_keyword_arguments():
+    x = torch.arange(4.0)
+    for out in (dispatch_probe(x, s=2.0), dispatch_probe(s=2.0, x=x)):
+        assert torch.equal(out[0], 2 * x) and not out[0].requires_grad
+    out = dispatch_probe(s=2.0, x=x.clone().requires_grad_())[0]
+    assert out.requires_grad
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        out.sum().backward()
+    with FakeTensorMode():
+        a = torch.empty(1, 4, 64, device="cuda", dtype=torch.bfloat16)
+        assert _native.sim_argmax(a=a, b=a, max_in_input_dtype=True)[0].dtype == torch.bfloat16
