@@ -291,7 +291,11 @@ def _rows_ok(t: torch.Tensor, align_elems: int) -> bool:
 # on a two-tensor op: 16 us a call through `torch.library.custom_op`, 6 us so;
 # a whole merge has six such calls and a model forward 450.
 
-_LIB = torch.library.Library("gpa", "FRAGMENT")
+# A second copy of this module in a process (loaded again, or under another
+# name) takes the registrations over; the first one's callables then run them.
+if "_library" in vars(torch.ops.gpa):
+    torch.ops.gpa._library._destroy()
+_LIB = torch.ops.gpa._library = torch.library.Library("gpa", "FRAGMENT")
 _Below = torch._C._AutoDispatchBelowAutograd
 
 
@@ -308,9 +312,10 @@ def _op(fn):
                            "formula was registered: the op is forward-only")
 
     torch.library.register_autograd(f"gpa::{name}", backward, lib=_LIB)
-    op = getattr(torch.ops.gpa, name).default
+    ops = torch.ops.gpa
 
     def call(*args, **kwargs):
+        op = getattr(ops, name).default
         if torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
                 isinstance(a, torch.Tensor) and a.requires_grad
                 for a in (*args, *kwargs.values()))):

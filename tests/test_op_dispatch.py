@@ -1,6 +1,8 @@
 """How the package's ops are dispatched (CPU): the callable that skips the
 autograd kernel and the registered op answer alike wherever a caller can tell
 them apart, on a small op registered the same way."""
+import subprocess
+import sys
 from typing import Tuple
 
 import pytest
@@ -61,3 +63,38 @@ def test_keyword_arguments():
     with FakeTensorMode():
         a = torch.empty(1, 4, 64, device="cuda", dtype=torch.bfloat16)
         assert _native.sim_argmax(a=a, b=a, max_in_input_dtype=True)[0].dtype == torch.bfloat16
+
+
+_TWO_COPIES = """
+import importlib, importlib.util, sys
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+sys.path.insert(0, {pkg!r})
+from merging import _native
+from merging.fused_similarity import fused_similarity_argmax
+spec = importlib.util.spec_from_file_location("another_native", _native.__file__)
+other = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(other)
+for again in (False, True):
+    if again:
+        importlib.reload(_native)
+    with FakeTensorMode():
+        a = torch.empty(1, 4, 64, device="cuda", dtype=torch.bfloat16)
+        for call in (_native.sim_argmax, other.sim_argmax, torch.ops.gpa.sim_argmax):
+            assert call(a, a)[1].shape == (1, 4)
+        assert fused_similarity_argmax(a, a)[0].dtype == torch.bfloat16
+    try:
+        other.sim_argmax(torch.zeros(1, 4, 64), torch.zeros(1, 4, 64))
+    except ValueError as e:
+        assert "GPU tensors" in str(e)
+    else:
+        raise AssertionError("a CPU tensor was taken")
+"""
+
+
+def test_two_copies_of_the_module_in_one_process():
+    """Loaded under a second name, then loaded again."""
+    script = _TWO_COPIES.format(pkg=str(_native.LIB_PATH.parents[2]))
+    done = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True,
+                          timeout=120)
+    assert done.returncode == 0, done.stderr
