@@ -518,25 +518,34 @@ extern "C" int gpa_merge_order(const int64_t* cell, int64_t frames, int64_t w, i
                                int64_t sy, int64_t num_special, int64_t* mask, int64_t* order,
                                void* stream) {
   gpa_clear_error();
-  if (frames < 0 || w < 0 || h < 0 || sx <= 0 || sy <= 0 || num_special < 0) {
+  // Without a cell no window is looked at, and of one frame every token is a
+  // destination: only the sizes that are used have to make sense.
+  const int64_t most = 0x7fffffff;
+  if (frames < 0 || (frames > 1 && num_special < 0) ||
+      (cell && (w < 0 || h < 0 || sx <= 0 || sy <= 0))) {
     gpa_set_error("gpa_merge_order: negative size or empty window");
     return GPA_E_INVALID;
   }
-  const int64_t tpi = w * h + num_special;
+  const bool fits = frames <= most && w <= most && w >= -most && h <= most && h >= -most &&
+                    num_special <= most && num_special >= -most && (!cell || (sx <= most && sy <= most));
+  const int64_t tpi = fits ? w * h + num_special : 0;
+  if (!fits || tpi > most) {
+    gpa_set_error("gpa_merge_order: %lld frames of %lld x %lld patches exceed the grid limit",
+                  (long long)frames, (long long)w, (long long)h);
+    return GPA_E_UNSUPPORTED;
+  }
+  if (tpi < 0) {
+    gpa_set_error("gpa_merge_order: negative frame size");
+    return GPA_E_INVALID;
+  }
   if (frames == 0 || tpi == 0) return GPA_OK;
   if (!mask || !order) {
     gpa_set_error("gpa_merge_order: null pointer");
     return GPA_E_INVALID;
   }
-  if (frames > 0x7fffffff || w > 0x7fffffff || h > 0x7fffffff || sx > 0x7fffffff || sy > 0x7fffffff ||
-      num_special > 0x7fffffff || tpi > 0x7fffffffLL) {
-    gpa_set_error("gpa_merge_order: %lld frames of %lld tokens exceed the grid limit",
-                  (long long)frames, (long long)tpi);
-    return GPA_E_UNSUPPORTED;
-  }
   OrderArgs a{};
-  a.hsy = (int)(h / sy);
-  a.wsx = (int)(w / sx);
+  a.hsy = cell ? (int)(h / sy) : 0;
+  a.wsx = cell ? (int)(w / sx) : 0;
   a.cell = a.hsy > 0 && a.wsx > 0 ? cell : nullptr;
   a.mask = mask;
   a.order = order;

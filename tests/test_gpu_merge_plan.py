@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from merging import _native  # noqa: F401  (registers the ops)
-from merging.merge import dst_mask, num_dst_tokens, window_cells
+from merging.merge import dst_mask, num_dst_tokens, token_merge_bipartite2d, window_cells
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +27,35 @@ def test_order_and_mask(dev, frames, w, h, sx, sy, ns, no_rand):
     assert torch.equal(got_mask, mask)
     assert torch.equal(got, torch.argsort(mask, stable=True))
     assert int((mask == -1).sum()) == num_dst_tokens(frames, w, h, sx, sy, ns, no_rand)
+
+
+@pytest.mark.parametrize("frames,w,h,sx,sy,ns,no_rand", [
+    (1, 6, 6, 0, 0, 5, False), (1, 6, 6, -1, 2, 5, False), (3, 6, 6, 0, 0, 5, True),
+    (3, 5, 7, 2, -3, 0, True), (1, 6, 6, 2, 2, -2, False), (1, -6, -6, 2, 2, 5, False),
+    (2, -6, -6, 2, 2, 5, True)])
+def test_sizes_that_no_window_uses(dev, frames, w, h, sx, sy, ns, no_rand):
+    """One frame, or no drawn patch: the windows are not looked at."""
+    mask = dst_mask(frames, w, h, sx, sy, ns, no_rand, None, dev)
+    got_mask, got = torch.ops.gpa.merge_order(None, frames, w, h, sx, sy, ns, dev)
+    assert torch.equal(got_mask, mask) and torch.equal(got, torch.argsort(mask, stable=True))
+    n = frames * (w * h + ns)
+    x = torch.randn(1, n, 256, device=dev)
+    m = token_merge_bipartite2d(x, w, h, sx, sy, 10, no_rand, num_special=ns)
+    assert torch.equal(m.index.mask, mask) and m.size.sum() == n
+
+
+def test_sizes_that_are_refused(dev):
+    cell = torch.zeros(2, 3, 3, device=dev, dtype=torch.int64)
+    mask = torch.empty(1, device=dev, dtype=torch.int64)
+    L = _native.lib()
+    for frames, w, h, sx, sy, ns, p, code in [
+            (-1, 6, 6, 2, 2, 5, 0, _native.GPA_E_INVALID), (3, 6, 6, 0, 2, 5, 1, _native.GPA_E_INVALID),
+            (3, -6, -6, 2, 2, 5, 1, _native.GPA_E_INVALID), (3, 6, 6, 2, 2, -1, 0, _native.GPA_E_INVALID),
+            (1, 6, -6, 2, 2, 5, 0, _native.GPA_E_INVALID),
+            (1, 2 ** 40, 2 ** 40, 2, 2, 5, 0, _native.GPA_E_UNSUPPORTED),
+            (1, 2 ** 16, 2 ** 16, 2, 2, 5, 0, _native.GPA_E_UNSUPPORTED)]:
+        assert L.gpa_merge_order(cell.data_ptr() if p else None, frames, w, h, sx, sy, ns,
+                                 mask.data_ptr(), mask.data_ptr(), None) == code
 
 
 @pytest.mark.parametrize("bad", [-1, 6, -2 ** 40, 2 ** 40])
