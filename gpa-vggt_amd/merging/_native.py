@@ -653,7 +653,7 @@ def merge_plan(node_max: torch.Tensor, node_idx: torch.Tensor, order: torch.Tens
     dev = _require_gpu(node_max, node_idx, order)
     B, ns = node_max.shape
     N = order.shape[0]
-    if node_max.dtype not in _DTYPE_CODES or node_idx.dtype != torch.int64 \
+    if (ns > 0 and node_max.dtype not in _DTYPE_CODES) or node_idx.dtype != torch.int64 \
             or order.dtype != torch.int64 or node_idx.shape != node_max.shape \
             or num_dst + ns != N or not 0 <= r <= ns:
         raise ValueError(f"gpa::merge_plan: node_max {node_max.dtype} {tuple(node_max.shape)}, "
@@ -671,9 +671,9 @@ def merge_plan(node_max: torch.Tensor, node_idx: torch.Tensor, order: torch.Tens
     ws = new(ws_bytes, dtype=torch.uint8) if ws_bytes else None
     with _on(dev):
         rc = L.gpa_merge_plan(
-            node_max.data_ptr(), _DTYPE_CODES[node_max.dtype], node_idx.data_ptr(), order.data_ptr(),
-            B, N, num_dst, r, edge.data_ptr(), dst_slot.data_ptr(), unm_abs.data_ptr(),
-            src_abs.data_ptr(), size.data_ptr(), offsets.data_ptr(), tokens.data_ptr(),
+            node_max.data_ptr(), _DTYPE_CODES.get(node_max.dtype, GPA_DTYPE_F32),   # (else empty)
+            node_idx.data_ptr(), order.data_ptr(), B, N, num_dst, r, edge.data_ptr(),
+            dst_slot.data_ptr(), unm_abs.data_ptr(), src_abs.data_ptr(), size.data_ptr(), offsets.data_ptr(), tokens.data_ptr(),
             ws.data_ptr() if ws is not None else None, ws_bytes, _stream(dev))
     _check(rc, "gpa::merge_plan")
     return edge, dst_slot, unm_abs, src_abs, size, offsets, tokens

@@ -128,3 +128,15 @@ def test_plan(dev, ns, num_dst, share, dtype, kind):
     for name, x, y in zip(("edge", "dst_slot", "unm_abs", "src_abs", "size", "offsets", "tokens"),
                           got, want):
         assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
+
+
+@pytest.mark.parametrize("metric_dim", [0, 128])
+def test_a_metric_of_another_type_without_sources(dev, metric_dim):
+    """One frame has no source: its maxima are an empty row of the metric's
+    type, which nothing reads; with sources the similarity refuses the type."""
+    x = torch.randn(2, 41, 256, device=dev, dtype=torch.float64)
+    m = token_merge_bipartite2d(x, 6, 6, 2, 2, 10, metric_dim=metric_dim)
+    assert torch.equal(m(x), x) and m.index.node_max.dtype == torch.float64
+    assert torch.equal(m.index.slot_tokens, torch.arange(41, device=dev).repeat(2))
+    with pytest.raises(ValueError):
+        token_merge_bipartite2d(x.view(1, 82, 256), 6, 6, 2, 2, 10, metric_dim=metric_dim)
