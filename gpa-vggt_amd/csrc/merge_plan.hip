@@ -13,27 +13,28 @@
 //   slots   = [sources past the first r of `edge`, in that order | destinations]
 //   lists   = per slot its own token, then the sources merged into it by
 //             increasing position (CSR offsets and tokens), and its size.
-// Both orders are stable sorts with 32-bit keys, done here as least
-// significant digit radix sorts of 8-bit digits: the maxima's bits in
-// descending order (four passes), and the merged rows' destinations (as many
-// passes as their count has bytes; rows come in increasing position, so
-// stability gives the order within a slot, and a slot of any length costs the
-// same).  A slot's list then starts at its own index plus the number of
-// merged rows with a smaller destination: a binary search in the sorted keys.
+// Both orders are stable sorts with 32-bit keys: the maxima's bits in
+// descending order, and the merged rows' destinations (rows come in increasing
+// position, so stability gives the order within a slot, and a slot of any
+// length costs the same).
 //
 // What bounds it: launches and latency, not bytes (137,400 tokens are 2 MB).
 // As torch operations this took over 60 launches per merge, three of them
-// merge sorts of up to 16 launches.  Up to kRankMax source rows both orders
-// come from counting: a row's rank is the number of rows before it, ns
-// compares per row spread over the whole chip, one launch for each order.
-// Above, each radix pass is two launches over kTile-row blocks (counts per
-// block, then a scatter in which every block sums the counts of the blocks
-// before it; that sum is ~50 rows of 1 KB at 200 frames, cheaper than a third
-// launch).
+// merge sorts of up to 16 launches.  Here, one of two ways (by_rank below):
+//   * Few rows: by counting.  A row's rank is the number of rows before it; the
+//     compares are spread over the whole chip, one launch for each order.  A
+//     slot's list starts at its own index plus the counted number of merged
+//     rows with a smaller destination.
+//   * More: least significant digit radix sorts of 8-bit digits (four passes
+//     for the maxima, as many for the destinations as their count has bytes).
+//     Each pass is two launches over kTile-row blocks (counts per block, then
+//     a scatter in which every block sums the counts of the blocks before it;
+//     that sum is ~50 rows of 1 KB at 200 frames, cheaper than a third
+//     launch), and a slot's start is a binary search in the sorted keys.
 // Measured, a whole merge with its K and V against the torch operations: 521
-// -> 169 us at 4 frames (70 -> 8 launches) with the plan's 38 us in one
-// workgroup, 12 us by counting since; 1,394 -> 1,085 us at 100 frames (83 ->
-// 21 launches; the order 5.5 us, the plan ~115 us of the GPU's time).
+// -> 121 us at 4 frames (70 -> 9 launches, the plan's two 6 us each), 1,394 ->
+// 1,085 us at 100 frames (83 -> 21 launches; the order 5.5 us, the plan ~115 us
+// of the GPU's time).
 #include "gpa_common.h"
 
 namespace gpa {
@@ -236,10 +237,21 @@ __device__ __forceinline__ uint32_t scan_digits(uint32_t x, uint32_t* part) {
 // the end are larger than any that is compared with them.
 constexpr int kRankRows = 16, kRankParts = 16, kRankThreads = kRankRows * kRankParts;
 constexpr int kRankKeys = 4096;
-// Where the two ways cross: the plan at 13,585 source rows takes 67 us by
-// counting and 84 us by radix passes, at 19,855 115 and 86 us (1,045: 8 and
-// 51 us; 3,135: 12 and 65 us; 7,315: 26 and 78 us).
-constexpr int kRankMax = 15360;
+// Where the two ways cross.  Counting costs a compare per pair of source rows,
+// half of one per pair of destination and source row, and ~1 ns per workgroup
+// (16 rows or destinations); the radix passes hardly more than their launches.
+// Microseconds, counting and radix passes (sources, destinations):
+//   B = 1   7,280, 3,677: 26, 82    15,600, 6,309: 82, 88    18,000, 1,400: 95, 87
+//   B = 2   9,360, 4,335: 63, 88    11,440, 4,993: 87, 88    13,520, 5,651: 116, 90
+//   B = 4   5,200, 3,019: 46, 85    7,280, 3,677: 71, 86     9,360, 4,335: 112, 88
+//   B = 16  2,080, 2,032: 34, 65    3,120, 2,361: 58, 73     4,160, 2,690: 100, 86
+//   B = 32  1,040, 1,703: 27, 60    2,080, 2,032: 60, 67     3,120, 2,361: 106, 75
+//   B = 128, 1,040, 1,703: 85, 66;  B = 300, 64, 20,000: 359, 98
+constexpr double kRankWork = 3.1e8;
+bool by_rank(int64_t B, int64_t ns, int64_t num_dst) {
+  const double n = (double)ns, d = (double)num_dst;
+  return ns == 0 || (double)B * (n * (n + d / 2) + 250.0 * (2 * n + d)) <= kRankWork;
+}
 
 // The sum over the parts of each row's counts, for the threads of part 0.
 __device__ __forceinline__ int sum_parts(int x, int (&part)[kRankParts][kRankRows + 1]) {
@@ -453,14 +465,14 @@ __global__ __launch_bounds__(kPlaceThreads) void plan_lists_kernel(PlanArgs a, c
   if (i == 0 && b == a.B - 1) a.offsets[a.B * (int64_t)(a.ns - a.r + a.num_dst)] = a.B * a.N;
 }
 
-size_t plan_ws_bytes(int64_t B, int64_t ns) {
-  if (ns <= kRankMax) return (size_t)B * ns * sizeof(uint32_t);
+size_t rank_ws_bytes(int64_t B, int64_t ns) { return (size_t)B * ns * sizeof(uint32_t); }
+size_t radix_ws_bytes(int64_t B, int64_t ns) {
   return (size_t)B * (4 * ns + (ns + kTile - 1) / kTile * kDigits) * sizeof(uint32_t);
 }
 
 template <typename T>
-void plan_launch(const PlanArgs& a, hipStream_t s) {
-  if (a.ns <= kRankMax) {
+void plan_launch(const PlanArgs& a, bool rank, hipStream_t s) {
+  if (rank) {
     const int row_blocks = (a.ns + kRankRows - 1) / kRankRows;
     const int dst_blocks = (a.num_dst + kRankRows - 1) / kRankRows;
     if (a.ns > 0)
@@ -568,7 +580,7 @@ extern "C" int gpa_merge_order(const int64_t* cell, int64_t frames, int64_t w, i
 
 extern "C" size_t gpa_merge_plan_workspace_bytes(int64_t B, int64_t num_src) {
   if (B <= 0 || num_src <= 0) return 0;
-  return plan_ws_bytes(B, num_src);
+  return radix_ws_bytes(B, num_src);     // either way's: the line depends on num_dst too
 }
 
 extern "C" int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t* node_idx,
@@ -602,7 +614,8 @@ extern "C" int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t
     gpa_set_error("%s: %lld x %lld tokens exceed the grid limit", fn, (long long)B, (long long)N);
     return GPA_E_UNSUPPORTED;
   }
-  const size_t need = plan_ws_bytes(B, ns);
+  const bool rank = by_rank(B, ns, num_dst);
+  const size_t need = rank ? rank_ws_bytes(B, ns) : radix_ws_bytes(B, ns);
   if (need && (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16)) {
     gpa_set_error("%s: 16-byte aligned workspace of %zu bytes required, %zu given", fn, need,
                   workspace ? workspace_bytes : (size_t)0);
@@ -631,7 +644,7 @@ extern "C" int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t
   while (a.passes < 4 && (top >> (8 * a.passes)) != 0) ++a.passes;
   a.blocks = (int)((ns + kTile - 1) / kTile);
   a.keys0 = (uint32_t*)workspace;
-  if (ns > kRankMax) {
+  if (!rank) {
     a.keys1 = a.keys0 + B * ns;
     a.vals0 = a.keys1 + B * ns;
     a.vals1 = a.vals0 + B * ns;
@@ -639,11 +652,11 @@ extern "C" int gpa_merge_plan(const void* node_max, int max_dtype, const int64_t
   }
   hipStream_t s = (hipStream_t)stream;
   if (max_dtype == GPA_DTYPE_F32)
-    plan_launch<float>(a, s);
+    plan_launch<float>(a, rank, s);
   else if (max_dtype == GPA_DTYPE_BF16)
-    plan_launch<__bf16>(a, s);
+    plan_launch<__bf16>(a, rank, s);
   else
-    plan_launch<_Float16>(a, s);
+    plan_launch<_Float16>(a, rank, s);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     gpa_set_error("%s: launch failed: %s", fn, hipGetErrorString(e));

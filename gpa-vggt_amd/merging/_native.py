@@ -673,7 +673,8 @@ def merge_plan(node_max: torch.Tensor, node_idx: torch.Tensor, order: torch.Tens
         rc = L.gpa_merge_plan(
             node_max.data_ptr(), _DTYPE_CODES.get(node_max.dtype, GPA_DTYPE_F32),   # (else empty)
             node_idx.data_ptr(), order.data_ptr(), B, N, num_dst, r, edge.data_ptr(),
-            dst_slot.data_ptr(), unm_abs.data_ptr(), src_abs.data_ptr(), size.data_ptr(), offsets.data_ptr(), tokens.data_ptr(),
+            dst_slot.data_ptr(), unm_abs.data_ptr(), src_abs.data_ptr(), size.data_ptr(),
+            offsets.data_ptr(), tokens.data_ptr(),
             ws.data_ptr() if ws is not None else None, ws_bytes, _stream(dev))
     _check(rc, "gpa::merge_plan")
     return edge, dst_slot, unm_abs, src_abs, size, offsets, tokens

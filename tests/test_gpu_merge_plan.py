@@ -1,7 +1,7 @@
 """The merge's bookkeeping kernels (gpa::merge_order, gpa::merge_plan) against
 torch's stable sorts: exact, every output.  Row counts sit at the edges of the
-counting path (up to 15,360 rows; 16 rows a workgroup, 4,096 keys staged at a
-time) and of the radix sort's blocks (4,096 rows);
+counting path (16 rows a workgroup, 4,096 keys staged at a time) and of the
+radix sort's blocks (4,096 rows), and on both sides of the line between them;
 maxima with ties, NaN, both zeros and infinities; all rows of a batch element
 in one slot; destination counts of one to three key bytes."""
 import pytest
@@ -128,6 +128,36 @@ def test_plan(dev, ns, num_dst, share, dtype, kind):
     for name, x, y in zip(("edge", "dst_slot", "unm_abs", "src_abs", "size", "offsets", "tokens"),
                           got, want):
         assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
+
+
+@pytest.mark.parametrize("B,ns,num_dst", [
+    (1, 15_360, 6234), (1, 16_500, 6234), (4, 7280, 3677), (4, 7900, 3900), (32, 2080, 2032),
+    (32, 2500, 2032), (128, 900, 1500), (128, 1040, 1703), (59, 17, 20_001), (60, 17, 20_002),
+    (300, 1, 5000), (40, 0, 40_000)])
+def test_both_sides_of_the_line_in_batches(dev, B, ns, num_dst):
+    """Counting on one side, radix passes on the other, down to one row each;
+    the workspace the entry point asks for is enough and no less is taken
+    than it needs."""
+    g = torch.Generator().manual_seed(B + ns)
+    node_max = (torch.randn(B, ns, generator=g) * 64).round() / 64          # ties
+    node_idx = torch.randint(0, num_dst, (B, ns), generator=g)
+    order = torch.randperm(num_dst + ns, generator=g)
+    order = torch.cat([order[:num_dst].sort().values, order[num_dst:].sort().values])
+    r = int(0.9 * ns + 0.5)
+    want = _expected(node_max, node_idx, order, num_dst, r)
+    got = torch.ops.gpa.merge_plan(node_max.to(dev), node_idx.to(dev), order.to(dev), num_dst, r)
+    for name, x, y in zip(("edge", "dst_slot", "unm_abs", "src_abs", "size", "offsets", "tokens"),
+                          got, want):
+        assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
+    if ns > 0:
+        L = _native.lib()
+        p = [x.data_ptr() for x in got]
+        x, i, o = node_max.to(dev), node_idx.to(dev), order.to(dev)
+        ws = torch.empty(B * ns * 4, device=dev, dtype=torch.uint8)
+        assert L.gpa_merge_plan_workspace_bytes(B, ns) >= ws.numel()
+        assert L.gpa_merge_plan(x.data_ptr(), _native.GPA_DTYPE_F32, i.data_ptr(), o.data_ptr(), B,
+                                num_dst + ns, num_dst, r, *p, ws.data_ptr(), ws.numel() - 4,
+                                None) == _native.GPA_E_WORKSPACE
 
 
 @pytest.mark.parametrize("metric_dim", [0, 128])
