@@ -6,7 +6,7 @@
 // wrapper reads it from q (:146, 177); VGGT uses 64, which the main kernel
 // serves.  Row sums add the fp32 P, as the reference's do (:113).
 //
-// Common to both kernels below
+// Common to the tiled and the narrow kernel below
 //   * Scores are computed transposed, S^T = K . Q^T, on v_mfma_f32_32x32x16
 //     (HD / 16 k-steps): a lane owns one query of a 32-query block and 16 of
 //     the tile's 32 keys (the other 16 sit in lane^32); the accumulator
@@ -34,7 +34,7 @@ namespace {
 
 constexpr int kAWaves = 4;
 constexpr int kAThreads = kAWaves * 64;
-constexpr int kAQ = kAWaves * 32;            // queries per workgroup (tiled kernel)
+constexpr int kAQ = kAWaves * 32;            // queries per workgroup (tiled and short kernels)
 constexpr int kAKT = 32;                      // keys per tile
 
 template <int KIND>
@@ -320,7 +320,184 @@ __global__ __launch_bounds__(kAThreads, HD >= 256 ? 1 : 2) void attn_tiled_kerne
 }
 
 // ---------------------------------------------------------------------------
-// Head dims 16 and 32: the narrow kernel.
+// Head dims 16 and 32, few keys or a small grid: one 32-query block per wave.
+//
+// What bounds such a call is its launches and one workgroup's walk over the
+// keys, not the chip.  So the bias is read where it lies (a pre-pass for it is
+// another launch, 2.5 us), a wave carries one block of 32 queries (with two,
+// half the waves do all the work of up to 128 queries), and the next tile's
+// loads wait in registers while a tile is computed: a two-slot LDS ring, K
+// row-major in padded rows, V transposed, each 16-key step's keys in the order
+// the score MFMA's result registers enumerate them.  The offset is the running
+// row max, O and the row sums rescaled on every tile.  At head dim 16 the P.V
+// product runs on a 32-feature block whose upper 16 features are zero.
+//
+// Against the narrow kernel below, microseconds (32 bf16, bias; heads x
+// queries, keys): 4 x 500, 64: 3.9 and 6.3; 16 x 1,374, 500: 12.7 and 15.6;
+// 1,703: 37.8 and 37.8; 16 x 2,748, 500: 15.3 and 16.1; 1,000: 27.2 and 25.7;
+// 128 x 1,374, 128: 12.7 and 13.4; 256: 21.0 and 19.6.
+
+// Position of key k (0..31) of a tile in the transposed V rows: step s =
+// k / 16 holds, in lane-half order, the keys the score MFMA's result
+// registers 8s .. 8s+7 of lanes 0-31 (hi = 0) and 32-63 (hi = 1) hold:
+// register r of half hi is key 8 (r / 4) + 4 hi + r % 4.
+__device__ __forceinline__ int vt_pos(int k) {
+  return (k & ~15) + ((k >> 2) & 1) * 8 + ((k >> 3) & 1) * 4 + (k & 3);
+}
+
+template <int HD, bool F16, int KIND>
+__global__ __launch_bounds__(kAThreads, 2) void attn_short_kernel(AnyDimArgs p) {
+  constexpr int KS = HD / 16;                 // k-steps of the score product
+  constexpr int DB = HD >= 32 ? HD / 32 : 1;  // 32-feature blocks of O
+  constexpr int KROW = HD + 8;                // padded K row (elements)
+  constexpr int VROW = kAKT + 8;              // padded transposed V row
+  constexpr int CH = HD / 8;                  // 16-byte chunks per key row
+  constexpr int NCH = kAKT * CH;              // chunks per tile and tensor
+  constexpr int CPT = (NCH + kAThreads - 1) / kAThreads;
+  __shared__ __attribute__((aligned(16))) uint16_t ks_lds[2][kAKT * KROW];
+  __shared__ __attribute__((aligned(16))) uint16_t vt_lds[2][DB * 32 * VROW];
+  __shared__ __attribute__((aligned(16))) float bias_lds[2][kAKT];
+
+  const int tid = threadIdx.x, lane = tid & 63, hi = lane >> 5, l32 = lane & 31;
+  const int wave = tid >> 6;
+  const int64_t bh = blockIdx.y, b = bh / p.H, h = bh % p.H;
+  const int64_t q_row = (int64_t)blockIdx.x * kAQ + wave * 32 + l32;
+  const uint16_t* Q = p.q + b * p.q_sb + h * p.q_sh;
+  const uint16_t* K = p.k + b * p.k_sb + h * p.k_sh;
+  const uint16_t* V = p.v + b * p.v_sb + h * p.v_sh;
+  const int64_t boff = b * p.bias_sb + h * p.bias_sh;
+  const float c = p.c;
+
+  if constexpr (HD == 16) {                   // the zero upper half of the O block
+    for (int i = tid; i < 2 * 32 * VROW; i += kAThreads) {
+      const int sl = i / (32 * VROW), r = i % (32 * VROW);
+      if (r >= 16 * VROW) vt_lds[sl][r] = 0;
+    }
+  }
+
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = q_row < p.M ? *reinterpret_cast<const bf16x8*>(Q + q_row * p.q_sm + 16 * ks + 8 * hi)
+                         : bf16x8{};
+
+  // One tile's K and V chunks and bias, into registers (zeros / -inf past N).
+  u32x4 kreg[CPT], vreg[CPT];
+  float breg = -INFINITY;
+  auto load_tile = [&](int t) {
+    const int64_t n0 = (int64_t)t * kAKT;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int cidx = tid + i * kAThreads;
+      const int key = cidx / CH, ch = cidx % CH;
+      const bool ok = cidx < NCH && n0 + key < p.N;
+      kreg[i] = ok ? *reinterpret_cast<const u32x4*>(K + (n0 + key) * p.k_sn + 8 * ch) : u32x4{};
+      vreg[i] = ok ? *reinterpret_cast<const u32x4*>(V + (n0 + key) * p.v_sn + 8 * ch) : u32x4{};
+    }
+    if (tid < kAKT)
+      breg = n0 + tid < p.N ? any_bias<KIND>(p.bias, boff + (n0 + tid) * p.bias_sn) * p.mul
+                            : -INFINITY;
+  };
+  auto store_tile = [&](int sl) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int cidx = tid + i * kAThreads;
+      if (cidx < NCH) {
+        const int key = cidx / CH, ch = cidx % CH;
+        *reinterpret_cast<u32x4*>(&ks_lds[sl][key * KROW + 8 * ch]) = kreg[i];
+        const int pos = vt_pos(key);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vt_lds[sl][(8 * ch + 2 * e) * VROW + pos] = (uint16_t)(vreg[i][e] & 0xffffu);
+          vt_lds[sl][(8 * ch + 2 * e + 1) * VROW + pos] = (uint16_t)(vreg[i][e] >> 16);
+        }
+      }
+    }
+    if (tid < kAKT) bias_lds[sl][tid] = breg;
+  };
+
+  float m = -1.0e30f, l = 0.f;                // finite: a tile of -inf biases scores 0
+  f32x16 o_acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o_acc[db] = f32x16{};
+
+  const int ntiles = (int)((p.N + kAKT - 1) / kAKT);
+  load_tile(0);
+  store_tile(0);
+  for (int t = 0; t < ntiles; ++t) {
+    const int sl = t & 1;
+    __syncthreads();                          // slot sl written; slot sl^1 free
+    if (t + 1 < ntiles) load_tile(t + 1);
+    // S^T = K . Q^T + bias / sm_scale
+    f32x16 sv;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 bv = *reinterpret_cast<const f32x4*>(&bias_lds[sl][8 * g + 4 * hi]);
+      sv[4 * g + 0] = bv[0];
+      sv[4 * g + 1] = bv[1];
+      sv[4 * g + 2] = bv[2];
+      sv[4 * g + 3] = bv[3];
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&ks_lds[sl][l32 * KROW + 16 * ks + 8 * hi]);
+      sv = mfma32x32x16_t<F16>(kf, qf[ks], sv);
+    }
+    // Online softmax: running max, rescale, P in the operand format.
+    float mx = sv[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sv[r]);
+    const float m_new = fmaxf(m, max_halves(mx) * c);
+    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
+    bf16x8 pb[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + e], c, -m));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[8 * s + e + 1], c, -m));
+        l += p0 + p1;
+        const bf16x2 pv2 = pack2<F16>(p0, p1);
+        pb[s][e] = pv2[0];
+        pb[s][e + 1] = pv2[1];
+      }
+    // O^T += V^T . P^T
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const bf16x8 vf =
+            *reinterpret_cast<const bf16x8*>(&vt_lds[sl][(db * 32 + l32) * VROW + 16 * s + 8 * hi]);
+        o_acc[db] = mfma32x32x16_t<F16>(vf, pb[s], o_acc[db]);
+      }
+    if (t + 1 < ntiles) store_tile(sl ^ 1);
+  }
+
+  const float l_tot = sum_halves(l);
+  if (q_row >= p.M) return;
+  const float inv = 1.0f / l_tot;
+  uint16_t* O = p.o + b * p.o_sb + h * p.o_sh + q_row * p.o_sm;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int f0 = db * 32 + 8 * g + 4 * hi;             // features f0 .. f0+3
+      if (f0 < HD) {
+        const bf16x2 lo = pack2<F16>(o_acc[db][4 * g + 0] * inv, o_acc[db][4 * g + 1] * inv);
+        const bf16x2 up = pack2<F16>(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
+        *reinterpret_cast<u32x2*>(O + f0) =
+            u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, up)};
+      }
+    }
+  if (p.lse && hi == 0) p.lse[b * p.lse_sb + h * p.lse_sh + q_row] = m + __log2f(l_tot);
+}
+
+// ---------------------------------------------------------------------------
+// Head dims 16 and 32, more than that: the narrow kernel.
 //
 // The VALU bounds it, not the matrix pipe: per wave and tile (64 queries x 32
 // keys) 32 exps, 32 FMAs, 32 row-sum adds, 16 packs and 16 max3 are ~870
@@ -571,8 +748,49 @@ __global__ __launch_bounds__(kAThreads, 3) void attn_narrow_kernel(AnyDimArgs p)
   }
 }
 
+// Whether the short kernel is the faster one at head dims 16 and 32.  Its line
+// in keys falls as the chip fills up: past four of its workgroups per CU its
+// slower tile counts from 192 keys on, past one from 512; below, a call is one
+// workgroup's walk and the other kernel's pre-pass and wider waves pay off only
+// from 2,048 keys (no bias and at most half the CUs busy: 4,096), or from 1,024
+// where many heads' K and V compete for the L2s.  Measured over 4 to 128 heads,
+// 1 to 8,000 queries and 32 to 20,000 keys in both formats: the kernel
+// taken is never over 1.14 times the better one's time, 1.002 times on average.
+bool short_call(const AnyDimArgs& a, int64_t D, int bias_kind) {
+  const int64_t groups = (a.M + kAQ - 1) / kAQ * a.BH;
+  if (groups > 1024) return a.N <= 192;
+  if (groups > 256) return a.N <= 512;
+  if (a.BH * D > 2048) return a.N <= 1024;
+  return a.N <= (bias_kind == GPA_BIAS_NONE && groups <= 128 ? 4096 : 2048);
+}
+
+template <int HD, bool F16>
+void launch_short(const AnyDimArgs& a, int bias_kind, hipStream_t s) {
+  const dim3 grid((unsigned)((a.M + kAQ - 1) / kAQ), (unsigned)(a.BH)), block(kAThreads);
+  switch (bias_kind) {
+    case GPA_BIAS_F32:
+      hipLaunchKernelGGL((attn_short_kernel<HD, F16, GPA_BIAS_F32>), grid, block, 0, s, a);
+      break;
+    case GPA_BIAS_BF16:
+      hipLaunchKernelGGL((attn_short_kernel<HD, F16, GPA_BIAS_BF16>), grid, block, 0, s, a);
+      break;
+    case GPA_BIAS_F16:
+      hipLaunchKernelGGL((attn_short_kernel<HD, F16, GPA_BIAS_F16>), grid, block, 0, s, a);
+      break;
+    default:
+      hipLaunchKernelGGL((attn_short_kernel<HD, F16, GPA_BIAS_NONE>), grid, block, 0, s, a);
+      break;
+  }
+}
+
 template <int HD, bool F16>
 hipError_t launch_hd(const AnyDimArgs& a, int bias_kind, hipStream_t s) {
+  if constexpr (HD < 64) {
+    if (short_call(a, HD, bias_kind)) {
+      launch_short<HD, F16>(a, bias_kind, s);
+      return hipGetLastError();
+    }
+  }
   const int64_t ntiles = (a.N + kAKT - 1) / kAKT, npad = ntiles * kAKT;
   const dim3 bgrid((unsigned)((npad + 255) / 256), (unsigned)a.BH), bblock(256);
   switch (bias_kind) {
