@@ -313,12 +313,16 @@ def _op(fn):
 
     torch.library.register_autograd(f"gpa::{name}", backward, lib=_LIB)
     ops = torch.ops.gpa
+    getattr(ops, name)                   # so that the namespace holds it
+    packets = vars(ops)
 
     def call(*args, **kwargs):
-        op = getattr(ops, name).default
-        if torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
+        if torch.compiler.is_compiling():
+            return getattr(ops, name).default(*args, **kwargs)
+        op = packets[name].default
+        if torch.is_grad_enabled() and any(
                 isinstance(a, torch.Tensor) and a.requires_grad
-                for a in (*args, *kwargs.values()))):
+                for a in ((*args, *kwargs.values()) if kwargs else args)):
             return op(*args, **kwargs)
         with _Below():
             return op(*args, **kwargs)
