@@ -182,19 +182,16 @@ __device__ __forceinline__ void place_member(const PlanArgs& a, int64_t b, int i
 
 // Ranks of a wave's items among its items of the same digit, in item order
 // (item u of all lanes before item u + 1), and the digit counts of the wave
-// in cnt (zeroed by the wave).  `live` marks the items that exist, all of them
-// below `items` (wave-uniform).
+// in cnt (zeroed by the wave).  `live` marks the items that exist.
 template <int ITEMS>
 __device__ __forceinline__ void wave_rank(const uint32_t (&digit)[ITEMS], const bool (&live)[ITEMS],
-                                          int items, uint32_t* cnt, uint32_t (&rank)[ITEMS]) {
+                                          uint32_t* cnt, uint32_t (&rank)[ITEMS]) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int d = 0; d < kDigits; d += 64) cnt[d + lane] = 0;
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int u = 0; u < ITEMS; ++u) {
-    rank[u] = 0;
-    if (u >= items) continue;
     uint64_t peers = __builtin_amdgcn_ballot_w64(live[u]);
 #pragma unroll
     for (int bit = 0; bit < 8; ++bit) {
@@ -416,7 +413,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(PlanArgs a, 
     sums[half][0][d] = before;
     sums[half][1][d] = all;
   }
-  wave_rank<kSortItems>(digit, live, kSortItems, cnt[wave], rank);
+  wave_rank<kSortItems>(digit, live, cnt[wave], rank);
   __syncthreads();
   uint32_t all = 0;
   if (tid < kDigits) {
