@@ -550,12 +550,12 @@ def main(argv=None) -> int:
         # (bf16, and fp32 k as the merged blocks keep it for the K merge).
         import gpa_aggregator as A
         qkv = (torch.randn(1, S * P, 3 * 1024, device=dev)).bfloat16()
-        ln_w = torch.ones(2, 64, device=dev)
-        ln_b = torch.zeros(2, 64, device=dev)
+        ln_w = torch.ones(64, device=dev, dtype=torch.bfloat16)      # as a block holds them
+        ln_b = torch.zeros(64, device=dev, dtype=torch.bfloat16)
         rope = A.Rope2D(100.0).table(A.frame_positions(37, pts, dev), 64)
         for k_f32, tag in ((False, "bf16"), (True, "k_f32")):
-            fn = lambda: torch.ops.gpa.qk_norm_rope(qkv, ln_w, ln_b, 1e-5, rope.pos, rope.cs,  # noqa: E731
-                                                    16, False, k_f32)
+            fn = lambda: _native.qk_norm_rope_params(qkv, ln_w, ln_w, ln_b, ln_b, 1e-5,  # noqa: E731
+                                                     rope.pos, rope.cs, 16, False, k_f32)
             fn()
             t = statistics.median(event_ms(fn, 5))
             nbytes = S * P * (2 * 1024 * 2 + 1024 * 2 + 1024 * (4 if k_f32 else 2))

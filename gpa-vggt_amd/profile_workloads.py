@@ -171,12 +171,13 @@ def main(argv=None) -> int:
     if which in ("qk", "all"):
         import gpa_aggregator as A
         qkv = torch.randn(1, 200 * 1374, 3 * 1024, device=dev).bfloat16()
-        ln_w, ln_b = torch.ones(2, 64, device=dev), torch.zeros(2, 64, device=dev)
+        ln_w = torch.ones(64, device=dev, dtype=torch.bfloat16)      # as a block holds them
+        ln_b = torch.zeros(64, device=dev, dtype=torch.bfloat16)
         rope = A.Rope2D(100.0).table(A.frame_positions(37, 5, dev), 64)
         for k_f32 in (False, True):
             for _ in range(reps):
-                torch.ops.gpa.qk_norm_rope(qkv, ln_w, ln_b, 1e-5, rope.pos, rope.cs, 16, False,
-                                           k_f32)
+                _native.qk_norm_rope_params(qkv, ln_w, ln_w, ln_b, ln_b, 1e-5, rope.pos, rope.cs,
+                                            16, False, k_f32)
         torch.cuda.synchronize()
         print(f"qk 274800 tokens x 16 heads (bf16 k, fp32 k) x {reps} done", flush=True)
         del qkv
