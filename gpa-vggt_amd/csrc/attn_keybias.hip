@@ -306,8 +306,9 @@ constexpr int kBoundWords = 4;
 // 1,703 keys 38.4 -> 36.7 us, 5,496 x 2,361 76.6 -> 75.4 us, 21,984 x 7,721
 // within 0.1 %.  It delays every workgroup a little, though, so the line lies
 // at two rounds of the chip's 512 places: 40 fp16 frames (3,840 workgroups of
-// 43 tiles) took 352 us so and take 348 us with the launch.  (The records and the bounds by one workgroup per head in one
-// launch took 6 us more than the two launches.)
+// 43 tiles) took 352 us so and take 348 us with the launch.  (The records and
+// the bounds by one workgroup per head in one launch took 6 us more than the
+// two launches.)
 constexpr int kFoldLoads = 4, kFoldTiles = 64 * kFoldLoads;
 constexpr int64_t kFoldGrid = 1024;
 __global__ __launch_bounds__(256) void row_bounds_kernel(const float* recs, float* bounds,

@@ -99,9 +99,9 @@ __global__ __launch_bounds__(kThreads, 1) void merge_metric_kernel(MetricArgs a)
 
   // The row of a block step.  kAhead: its index is fetched two steps before its
   // loads are issued, so that these never wait for it; otherwise with them.
-  // Ahead costs registers, which the widest fp32 rows do not have: at C = 1024
-  // the fp32 loads then wait on the moves around them, and the fp16 projection
-  // spills.  Microseconds with the loads and ahead, 137,400 rows:
+  // Ahead costs registers, which the widest fp32 rows do not have (248 to 254
+  // VGPRs at C = 1024; the fp16 projection spills).  Microseconds with the
+  // loads and ahead, 137,400 rows:
   //            C = 256        512            768            1024
   //   bf16     65.0 / 59.5    72.6 / 68.3    79.9 / 75.5    94.4 / 89.9
   //   fp32     67.5 / 61.3    81.3 / 78.8    112.5 / 107.5  137.1 / 142.8

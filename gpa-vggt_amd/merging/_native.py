@@ -9,6 +9,11 @@ the custom ops:
     gpa::sim_argmax(Tensor a, Tensor b) -> (Tensor max_f32, Tensor idx_i64)
     gpa::attn_keybias(Tensor q, Tensor k, Tensor v, Tensor? bias,
                       float sm_scale, bool return_lse) -> (Tensor o, Tensor lse)
+    gpa::attn_keybias_rows(Tensor q, Tensor k, Tensor v, Tensor? bias,
+                           float sm_scale) -> Tensor rows
+    gpa::attn_keybias_join(Tensor q, Tensor k, Tensor v, Tensor? bias,
+                           float sm_scale, Tensor other_o, Tensor other_lse,
+                           int frames) -> Tensor rows
     gpa::merge_heads(Tensor t, Tensor offsets, Tensor tokens, int slots,
                      bool mean) -> (Tensor out, Tensor size, Tensor log_size)
     gpa::merge_order(Tensor? cell, int frames, int w, int h, int sx, int sy,
@@ -21,9 +26,21 @@ the custom ops:
     gpa::qk_norm_rope(Tensor qkv, Tensor ln_w, Tensor ln_b, float eps,
                       Tensor? pos, Tensor? rope_cs, int heads, bool q_f32,
                       bool k_f32) -> (Tensor q, Tensor k)
+    gpa::qk_norm_rope_params(Tensor qkv, Tensor q_w, Tensor k_w, Tensor q_b,
+                             Tensor k_b, float eps, Tensor? pos, Tensor? rope_cs,
+                             int heads, bool q_f32, bool k_f32)
+                             -> (Tensor q, Tensor k)
     gpa::pool_shared(Tensor k, Tensor v, int frames, int pts, int grid_h,
                      int grid_w, int kp, bool want_assign)
                      -> (Tensor pk, Tensor pv, Tensor size, Tensor assign)
+    gpa::shared_set(Tensor k, Tensor v, int frames, int pts, int grid_h,
+                    int grid_w, int kp)
+                    -> (Tensor k, Tensor v, Tensor bias, Tensor size)
+    gpa::merge_metric(Tensor metric, Tensor proj, Tensor? order, int mode)
+                      -> Tensor operands
+    gpa::residual_layernorm(Tensor x, Tensor? y, Tensor? gamma, Tensor? weight,
+                            Tensor? bias, float eps, bool want_h)
+                            -> (Tensor h, Tensor ln)
 
 All launch on torch's current stream of the input's device.  There is no
 fallback: a missing library or a non-GPU tensor raises.
@@ -222,8 +239,8 @@ def exported_symbols() -> Tuple[str, ...]:
             "gpa_pool_shared_bf16", "gpa_merge_metric_bf16", "gpa_sim_argmax_f16",
             "gpa_attn_keybias_f16", "gpa_residual_layernorm_bf16",
             "gpa_attn_keybias_bf16_noalloc", "gpa_lse_combine_f16", "gpa_qk_norm_rope_f16",
-            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16", "gpa_shared_set", "gpa_attn_keybias_join",
-            "gpa_qk_norm_rope_params")
+            "gpa_residual_layernorm_f16", "gpa_pool_shared_f16", "gpa_shared_set",
+            "gpa_attn_keybias_join", "gpa_qk_norm_rope_params")
 
 
 def _check(rc: int, what: str) -> None:

@@ -88,6 +88,9 @@ def dst_mask(num_imgs: int, w: int, h: int, sx: int, sy: int, num_special: int,
     laid out with row length (w//sx)*sx over the first (h//sy)*sy*(w//sx)*sx
     patch positions of the frame; `no_rand=True` marks no patch of frames
     >= 1 (reference :105-118 writes an all-zero pattern).
+
+    The rules restated in torch ops, on any device: a merge takes mask and
+    order from `gpa::merge_order`, which is tested against this.
     """
     tpi = w * h + num_special
     n = num_imgs * tpi

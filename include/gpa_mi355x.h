@@ -1,8 +1,8 @@
 /*
  * gpa_mi355x.h — C ABI of the MI355X (gfx950) GPA-VGGT merging hot path.
  *
- * Ten entry points (two of them with an fp16 twin, the attention also
- * with an allocation-free variant) sit behind this boundary:
+ * The operations behind this boundary (most with an fp16 twin, the
+ * attention also with an allocation-free variant):
  *
  *   gpa_sim_argmax_bf16   — fused cosine-similarity row max / argmax between
  *                           source and destination token metrics
@@ -11,6 +11,9 @@
  *   gpa_attn_keybias_bf16 — flash attention with a per-key additive bias
  *                           (replaces merging/fused_attention.py:130-180,
  *                            the Triton `_attn_keybias_kernel` at :70-127).
+ *   gpa_attn_keybias_join — the same attention, joined in its epilogue with one
+ *                           over further keys by their log2 LSE (the split
+ *                           path of vggt/layers/attention.py:148-176).
  *   gpa_merge_heads       — deterministic segmented mean/sum of token rows,
  *                           the K/V merge (replaces the scatter_reduce_ of
  *                           merging/merge.py:234-250).
@@ -21,9 +24,13 @@
  *                           LSE (replaces vggt/layers/attention.py:166-176).
  *   gpa_qk_norm_rope_bf16 (and _f16) — qk LayerNorm + 2D RoPE + cast of a block's
  *                           attention operands (replaces the torch op
- *                           sequence of vggt/layers/attention.py:210-220).
+ *                           sequence of vggt/layers/attention.py:210-220);
+ *                           gpa_qk_norm_rope_params takes the four LayerNorm
+ *                           parameters where and as the model holds them.
  *   gpa_pool_shared_bf16 (and _f16) — pooled summaries of the frame-special shared
- *                           K/V set (replaces vggt/layers/attention.py:113-140).
+ *                           K/V set (replaces vggt/layers/attention.py:113-140);
+ *                           gpa_shared_set writes the whole set: special
+ *                           tokens, summaries and bias.
  *   gpa_merge_metric_bf16 — the merge's metric projection, normalisation and
  *                           dst/src split (replaces merging/merge.py:180-187).
  *   gpa_residual_layernorm_bf16 (and _f16) — residual + LayerScale + LayerNorm of the

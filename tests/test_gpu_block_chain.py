@@ -1,7 +1,8 @@
 """Blocks run as a chain (the last residual pass also writes the next block's
 LayerNorm) against the same blocks called one by one: bit for bit, and a block
 with a forward hook, a replaced forward or another dtype is called as a
-module, its hook seeing and able to change what passes.  The LayerNorm
+module, its hook seeing and able to change what passes (everything else that
+takes a block out of the chain: test_block_chain.py, on the CPU).  The LayerNorm
 parameters of the qk norm in each format against the stacked fp32 ones."""
 import pytest
 import torch

@@ -3,8 +3,10 @@
 * The C-ABI library loads and exports every function `include/gpa_mi355x.h`
   declares; argument validation returns the documented error codes before
   any device work.
-* The product's host logic (`merging.merge.dst_mask`, `num_dst_tokens`)
-  agrees with the oracle's step-by-step restatement of merging/merge.py.
+* The destination rules as torch ops (`merging.merge.dst_mask`, which the
+  merge's kernel is tested against on the GPU) and their closed-form count
+  (`num_dst_tokens`, which the merge runs) agree with the oracle's
+  step-by-step restatement of merging/merge.py.
 * The Python entry points refuse CPU tensors loudly (there is no CPU path).
 """
 import ctypes
