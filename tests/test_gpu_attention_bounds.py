@@ -1,5 +1,5 @@
-"""Head dim 64 on both sides of the line where the attention forms its row
-bounds itself (8,192 keys): certified, tile-0 and lazily moved offsets (logit
+"""Head dim 64 on both sides of the lines up to which the attention forms its row
+bounds itself (8,192 keys, 1,024 workgroups): certified, tile-0 and lazily moved offsets (logit
 scales from 0.3 to 30), an outlier key in the first and in the last tile.
 
 Bar: a row's relative error within 16-bit P and output, 4 * 2^-9 (bf16) or
@@ -66,3 +66,19 @@ def test_last_tile_without_bias(dev, N, join):
         assert (lse.cpu() - ref_lse).abs().max().item() <= 2.0 ** -8 / 0.6931   # bf16 P in the sum
     rel = (o.float().cpu() - ref).norm(dim=-1) / ref.norm(dim=-1)
     assert rel.max().item() <= 4 * 2.0 ** -9, rel.max().item()
+
+
+@pytest.mark.parametrize("dtype,ulp", [(torch.bfloat16, 2.0 ** -9), (torch.float16, 2.0 ** -12)])
+@pytest.mark.parametrize("B,H", [(64, 16), (205, 5)])
+@pytest.mark.parametrize("scale", [0.3, 3.0])
+def test_both_sides_of_the_grid_line(dev, dtype, ulp, B, H, scale):
+    """1,024 and 1,025 workgroups: bounds formed in the kernel, and by a launch."""
+    g = torch.Generator(device=dev).manual_seed(B)
+    q, k, v = (torch.randn(B, H, t, 64, device=dev, generator=g) for t in (100, 301, 301))
+    q, k, v = (q * scale).to(dtype), (k * scale).to(dtype), v.to(dtype)
+    bias = torch.randint(1, 9, (B, 1, 1, 301), device=dev, generator=g).float().log().to(dtype)
+    o = attention_keybias(q, k, v, bias.expand(B, H, 1, 301), 0.125)
+    x = q.double() @ k.double().transpose(-1, -2).contiguous() * 0.125 + bias.double()
+    ref = torch.softmax(x, -1) @ v.double()
+    rel = (o.double() - ref).norm(dim=-1) / ref.norm(dim=-1)
+    assert rel.max().item() <= 4 * ulp, rel.max().item()
