@@ -136,8 +136,8 @@ int gpa_sim_argmax_f16(const void* a, const void* b,
  * 16 bytes of row maxima and means, and one flag byte per 64 queries.  The
  * reference wrapper allocates the analogous padded bias buffer
  * (merging/fused_attention.py:159-160).  At head dims other than 64 the call
- * writes one fp32 bias row per (batch, head) there instead (4 bytes per key,
- * rounded up to 32 keys), which the same size holds. */
+ * writes at most one fp32 bias row per (batch, head) there instead (4 bytes per
+ * key, rounded up to 32 keys), which the same size holds. */
 size_t gpa_attn_keybias_workspace_bytes(int64_t B, int64_t H, int64_t M, int64_t N);
 
 /*
@@ -145,8 +145,9 @@ size_t gpa_attn_keybias_workspace_bytes(int64_t B, int64_t H, int64_t M, int64_t
  * 256} (the reference kernel's HEAD_DIM, fused_attention.py:82, 97, 177).
  * D = 64 (VGGT) runs the tuned kernel with a certified fixed softmax
  * offset; D = 128 and 256 a tiled kernel with a lazily moved offset, D = 16
- * and 32 a kernel of two query blocks per wave with the exact running max,
- * all with the same contract.
+ * and 32 a kernel of two query blocks per wave with the exact running max, or
+ * with few keys or on a small grid one of one block per wave, all with the same
+ * contract.
  *   o[b,h,m,:] = softmax_n( q[b,h,m,:].k[b,h,n,:] * sm_scale + bias[b,h,n] ) . v[b,h,n,:]
  *   lse[b,h,m] = log2( sum_n 2^( (q.k*sm_scale + bias) * log2(e) ) )   (if lse != NULL)
  * Replaces merging/fused_attention.py:130-180 (`attention_keybias`) and the
@@ -280,7 +281,8 @@ int gpa_merge_order(const int64_t* cell, int64_t frames, int64_t w, int64_t h,
                     int64_t sx, int64_t sy, int64_t num_special,
                     int64_t* mask, int64_t* order, void* stream);
 
-/* Bytes of device workspace gpa_merge_plan needs (16-byte aligned). */
+/* Bytes of device workspace that is enough for gpa_merge_plan with any num_dst
+ * (16-byte aligned). */
 size_t gpa_merge_plan_workspace_bytes(int64_t B, int64_t num_src);
 
 /*
