@@ -1,4 +1,4 @@
-"""The torch.library registration of every custom op: `torch.library.opcheck`
+"""The torch.library registration of the custom ops: `torch.library.opcheck`
 (schema, fake implementation against the real op's outputs, AOT dispatch
 with dynamic shapes) on small inputs, and a compiled graph (fullgraph,
 `aot_eager`, which traces through the fake implementations and generates
@@ -91,3 +91,32 @@ def test_compiled_graph_matches_eager(dev):
     for e, c in zip(eager, compiled):
         assert e.dtype == c.dtype and e.shape == c.shape
         assert torch.equal(e, c)
+
+
+def _new_op_cases(dev):
+    """The ops that the merge's bookkeeping and the blocks use besides (rows, join
+    and the shared set: test_gpu_attention_join.py)."""
+    g = _g(2)
+    frames, P = 3, 41
+    cell = torch.randint(0, 4, (frames - 1, 3, 3), device=dev, generator=g)
+    _, order = torch.ops.gpa.merge_order(cell, frames, 6, 6, 2, 2, 5, dev)
+    num_dst = P + (frames - 1) * (5 + 9)
+    ns = frames * P - num_dst
+    node_max = torch.randn(2, ns, device=dev, generator=g)
+    node_idx = torch.randint(0, num_dst, (2, ns), device=dev, generator=g)
+    qkv = torch.randn(1, frames * P, 3 * 2 * 64, device=dev, generator=g).bfloat16()
+    w = torch.randn(64, device=dev, generator=g).bfloat16()
+    rope = A.Rope2D(100.0).table(A.frame_positions(6, 5, dev), 64)
+    return {
+        "merge_order": (cell, frames, 6, 6, 2, 2, 5, dev),
+        "merge_order_no_cell": (None, frames, 6, 6, 2, 2, 5, dev),
+        "merge_plan": (node_max, node_idx, order, num_dst, ns // 2),
+        "qk_norm_rope_params": (qkv, w, w, w, w, 1e-6, rope.pos, rope.cs, 2, False, True),
+    }
+
+
+@pytest.mark.parametrize("case", ["merge_order", "merge_order_no_cell", "merge_plan",
+                                  "qk_norm_rope_params"])
+def test_opcheck_of_the_blocks_and_the_merge(dev, case):
+    op = getattr(torch.ops.gpa, case.replace("_no_cell", ""))
+    torch.library.opcheck(op, _new_op_cases(dev)[case])
