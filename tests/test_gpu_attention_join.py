@@ -13,7 +13,8 @@ import torch
 
 import gpa_aggregator as A
 from merging import _native
-from merging.fused_attention import attention_join, attention_keybias, attention_rows
+from merging.fused_attention import (attention_join, attention_keybias, attention_rows,
+                                     combine_by_lse)
 from oracle.attention import attention_reference, lse_combine
 
 pytestmark = pytest.mark.gpu
@@ -106,3 +107,29 @@ def test_opcheck(dev):
         q, k, k, None, 0.125, q.view(2, 3, 41, 64).transpose(0, 1).contiguous(),
         torch.zeros(3, 2, 41, device=dev), 3))
     assert A.pool_kernel_applies(q, 6, 6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S,H,P,n_own,n", [(4, 4, 206, 201, 120), (16, 2, 1374, 1369, 480)])
+def test_join_is_no_further_from_64_bits_than_its_parts(dev, dtype, S, H, P, n_own, n):
+    """The join rounds the shared half once less than the two calls and
+    `combine_by_lse`, so its output differs from theirs, repeats itself exactly
+    and lies no further from the softmax over both key sets in 64 bits."""
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, sk, sv = (torch.randn(1, H, t, 64, device=dev, generator=g).to(dtype)
+                 for t in (S * P, n, n))
+    ok, ov = (torch.randn(S, H, n_own, 64, device=dev, generator=g).to(dtype) for _ in "kv")
+    bias = torch.randint(1, 60, (1, H, 1, n), device=dev, generator=g).float().log().to(dtype)
+    q_f = q.view(H, S, P, 64).transpose(0, 1).contiguous()
+    own, own_lse = attention_keybias(q_f, ok, ov, None, 0.125, return_lse=True)
+    got = attention_join(q, sk, sv, bias, 0.125, own, own_lse, S)
+    assert torch.equal(got, attention_join(q, sk, sv, bias, 0.125, own, own_lse, S))
+    shared, shared_lse = attention_keybias(q, sk, sv, bias, 0.125, return_lse=True)
+    parts = combine_by_lse(own, own_lse, shared, shared_lse, S)
+    keys = torch.cat((ok, sk.expand(S, H, n, 64)), 2).double().transpose(-1, -2).contiguous()
+    values = torch.cat((ov, sv.expand(S, H, n, 64)), 2).double()
+    x = q_f.double() @ keys * 0.125
+    x[..., n_own:] += bias.double()
+    ref = (torch.softmax(x, -1) @ values).permute(0, 2, 1, 3).reshape(1, S * P, H * 64)
+    err, err_parts = ((t.double() - ref).norm().item() for t in (got, parts))
+    assert err <= err_parts
